@@ -44,130 +44,184 @@ __device__ inline cdbl cexp_d(double re, double im)
     return {e * cs, e * sn};
 }
 
-// single / double layer kernels, potential.h:22-47
-__device__ inline cdbl layer64(d3 src, d3 trg, d3 n, double kr, double ki, int type)
+// 1 / d for quotients that share the denominator d: the reciprocal estimate and two Newton steps,
+// then per quotient the product, its residual and the correction. These are the steps of the
+// compiler's own FP64 division without its range scaling, so the quotients are its bits (the
+// correctly rounded ones) as long as neither operand nor quotient comes near the exponent limits;
+// layer64_pair checks that and divides plainly otherwise.
+__device__ inline double shared_rcp(double d)
 {
-    if (type == 0)
-    {
-        d3 s = trg - src;
-        double r2 = dotd(s, s);
-        if (r2 == 0)
-            return {0, 0};
-        double r = sqrt(r2);
-        cdbl e = cexp_d(-r * ki, r * kr);
-        double q = 4 * PI_R * r;
-        return {e.re / q, e.im / q};
-    }
-    d3 s = src - trg;
-    double r2 = dotd(s, s);
-    if (r2 == 0)
-        return {0, 0};
-    double r = sqrt(r2);
-    double zr = -r * ki, zi = r * kr;
-    cdbl e = cexp_d(zr, zi);
-    double q = 4 * PI_R * r2 * r;
-    double ar = -e.re / q, ai = -e.im / q;
-    double br = 1 - zr, bi = -zi;
-    double pr = ar * br - ai * bi, pi = ar * bi + ai * br;
-    double dn = dotd(s, n);
-    return {pr * dn, pi * dn};
+    double y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+    return __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+}
+__device__ inline double shared_div(double n, double d, double y)
+{
+    const double m = n * y;
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d, m, n), y, m), d, n);
 }
 
-
-// singular_point (integrand.h:52-147); trial = tv, test = sv
-__device__ inline cdbl sing_point64(double xsi, double e1, double e2, double e3, double w, const d3 *tv,
-                                    const d3 *sv, d3 tn, int nn, double kr, double ki, int type)
+// single / double layer kernels (potential.h:22-47) of one (source point, target) pair, split in
+// two: the part without the wave number, computed once for the 9 wave numbers (r = |trg - src|,
+// the denominators 4 pi r and 4 pi r^2 r with their shared reciprocals, and (src - trg) . n),
+// and the part per wave number, whose complex exponential serves both layers. r = 0: the target
+// is the source point and both kernels are 0. y0 = 0: the denominators are divided by plainly.
+struct LayerTarget
 {
-    double rr = 0, ri = 0;
-    xsi = 0.5 * (xsi + 1);
-    e1 = 0.5 * (e1 + 1);
-    e2 = 0.5 * (e2 + 1);
-    e3 = 0.5 * (e3 + 1);
-    double jw = 0;
-#define ADD(A, Bp, F)                                      \
-    {                                                      \
-        cdbl g_ = layer64((A), (Bp), tn, kr, ki, type);    \
-        rr += g_.re * (F);                                 \
-        ri += g_.im * (F);                                 \
+    double r, q0, y0, q1, y1, dn;
+};
+__device__ inline LayerTarget layer_target(d3 src, d3 trg, d3 n)
+{
+    const d3 s0 = trg - src;
+    const double r2 = dotd(s0, s0);
+    if (r2 == 0)
+        return {0, 0, 0, 0, 0, 0};
+    const double r = sqrt(r2);
+    const d3 s1 = src - trg;  // = -s0 exactly, so dotd(s1, s1) == r2
+    const double q0 = 4 * PI_R * r, q1 = 4 * PI_R * r2 * r;
+    const bool plain = !(r > 1e-60 && r < 1e60);
+    return {r, q0, plain ? 0.0 : shared_rcp(q0), q1, plain ? 0.0 : shared_rcp(q1), dotd(s1, n)};
+}
+// e^(x + i y) for |x| < 600 and |y| < 2^19: det_exp and det_sincos (detmath.hpp) without their
+// branches, so that the three polynomial chains run side by side. Same operations on the same
+// operands: the rounding adds a half of x's sign before it truncates (only the sign of a zero
+// differs, which neither result sees), the scaling by 2^k cannot leave the normal range, and the
+// quadrant picks and negates.
+__device__ inline double round_half_away_b(double x) { return __builtin_trunc(x + __builtin_copysign(0.5, x)); }
+__device__ inline cdbl cexp_mid(double x, double y)
+{
+    using namespace detm;
+    const double kd = round_half_away_b(x * INV_LN2), qd = round_half_away_b(y * TWO_OVER_PI);
+    const double t = (x - kd * LN2_HI) - kd * LN2_LO;
+    const double r = ((y - qd * PIO2_1) - qd * PIO2_2) - qd * PIO2_3;
+    const double z = r * r;
+    double p = F13, ps = F17, pc = F16;
+    p = F12 + t * p, ps = F15 - z * ps, pc = F14 - z * pc;
+    p = F11 + t * p, ps = F13 - z * ps, pc = F12 - z * pc;
+    p = F10 + t * p, ps = F11 - z * ps, pc = F10 - z * pc;
+    p = F9 + t * p, ps = F9 - z * ps, pc = F8 - z * pc;
+    p = F8 + t * p, ps = F7 - z * ps, pc = F6 - z * pc;
+    p = F7 + t * p, ps = F5 - z * ps, pc = F4 - z * pc;
+    p = F6 + t * p, ps = F3 - z * ps, pc = F2 - z * pc;
+    p = F5 + t * p;
+    p = F4 + t * p;
+    p = F3 + t * p;
+    p = F2 + t * p;
+    p = 1.0 + t * p;
+    p = 1.0 + t * p;
+    const double e = __builtin_ldexp(p, (int)kd);
+    const double sr = r - (r * z) * ps, cr = 1.0 - z * pc;
+    const int q = (int)qd;
+    const double s0 = q & 1 ? cr : sr, c0 = q & 1 ? sr : cr;
+    return {e * ((q + 1) & 2 ? -c0 : c0), e * (q & 2 ? -s0 : s0)};
+}
+__device__ inline void layer64_pair(const LayerTarget &t, double kr, double ki, cdbl &g0, cdbl &g1)
+{
+    const double zr = -t.r * ki, zi = t.r * kr;
+    double ar, ai;
+    if (t.y0 != 0 && fabs(zr) < 600.0 && fabs(zi) < 5e5)  // |e^z| and its parts stay above 2^-930
+    {
+        const cdbl e = cexp_mid(zr, zi);
+        g0 = {shared_div(e.re, t.q0, t.y0), shared_div(e.im, t.q0, t.y0)};
+        ar = -shared_div(e.re, t.q1, t.y1);
+        ai = -shared_div(e.im, t.q1, t.y1);
     }
+    else if (t.r == 0)
+    {
+        g0 = g1 = {0, 0};
+        return;
+    }
+    else
+    {
+        const cdbl e = cexp_d(zr, zi);
+        g0 = {e.re / t.q0, e.im / t.q0};
+        ar = -e.re / t.q1;
+        ai = -e.im / t.q1;
+    }
+    const double br = 1 - zr, bi = -zi;
+    const double pr = ar * br - ai * bi, pi = ar * bi + ai * br;
+    g1 = {pr * t.dn, pi * t.dn};
+}
+
+// Region maps of the singular rules, singular_point (integrand.h:52-147): local coordinates of
+// region `sub` on the trial triangle (ta, tb) and the test triangle (sa, sb), and the factor f of
+// its term. nn = common vertices (3: 6 regions, 2: 5, 1: 2).
+__device__ inline int sing_regions(int nn) { return nn == 3 ? 6 : nn == 2 ? 5 : nn == 1 ? 2 : 0; }
+__device__ inline void sing_map(int nn, int sub, double xsi, double e1, double e2, double e3, double &ta, double &tb,
+                                double &sa, double &sb, double &f)
+{
+    const double e12 = e1 * e2, e123 = e1 * e2 * e3;
+    // the two ends of a region; odd regions of nn == 3 swap the triangles' roles
+    double a0, a1, b0, b1;
+    bool swap = false;
+    f = 1.0;
     if (nn == 3)
     {
-        jw = xsi * xsi * xsi * e1 * e1 * e2;
-        double e12 = e1 * e2, e123 = e1 * e2 * e3;
-        ADD(l2g2(xsi, xsi * (1.0 - e1 + e12), tv), l2g2(xsi * (1.0 - e123), xsi * (1.0 - e1), sv), 1.0);
-        ADD(l2g2(xsi * (1.0 - e123), xsi * (1.0 - e1), tv), l2g2(xsi, xsi * (1.0 - e1 + e12), sv), 1.0);
-        ADD(l2g2(xsi, xsi * (e1 - e12 + e123), tv), l2g2(xsi * (1.0 - e12), xsi * (e1 - e12), sv), 1.0);
-        ADD(l2g2(xsi * (1.0 - e12), xsi * (e1 - e12), tv), l2g2(xsi, xsi * (e1 - e12 + e123), sv), 1.0);
-        ADD(l2g2(xsi * (1.0 - e123), xsi * (e1 - e123), tv), l2g2(xsi, xsi * (e1 - e12), sv), 1.0);
-        ADD(l2g2(xsi, xsi * (e1 - e12), tv), l2g2(xsi * (1.0 - e123), xsi * (e1 - e123), sv), 1.0);
+        swap = (sub & 1) != 0;
+        a0 = xsi;
+        if (sub < 2)
+        {
+            a1 = xsi * (1.0 - e1 + e12);
+            b0 = xsi * (1.0 - e123);
+            b1 = xsi * (1.0 - e1);
+        }
+        else if (sub < 4)
+        {
+            a1 = xsi * (e1 - e12 + e123);
+            b0 = xsi * (1.0 - e12);
+            b1 = xsi * (e1 - e12);
+        }
+        else
+        {
+            swap = !swap;
+            a1 = xsi * (e1 - e12);
+            b0 = xsi * (1.0 - e123);
+            b1 = xsi * (e1 - e123);
+        }
     }
     else if (nn == 2)
     {
-        jw = xsi * xsi * xsi * e1 * e1;
-        double e12 = e1 * e2, e123 = e1 * e2 * e3;
-        ADD(l2g2(xsi, xsi * e1 * e3, tv), l2g2(xsi * (1.0 - e12), xsi * e1 * (1.0 - e2), sv), 1.0);
-        ADD(l2g2(xsi, xsi * e1, tv), l2g2(xsi * (1.0 - e123), xsi * e1 * e2 * (1 - e3), sv), e2);
-        ADD(l2g2(xsi * (1.0 - e12), xsi * e1 * (1.0 - e2), tv), l2g2(xsi, xsi * e123, sv), e2);
-        ADD(l2g2(xsi * (1.0 - e123), xsi * e12 * (1.0 - e3), tv), l2g2(xsi, xsi * e1, sv), e2);
-        ADD(l2g2(xsi * (1.0 - e123), xsi * e1 * (1.0 - e2 * e3), tv), l2g2(xsi, xsi * e12, sv), e2);
-    }
-    else if (nn == 1)
-    {
-        jw = xsi * xsi * xsi * e2;
-        ADD(l2g2(xsi, xsi * e1, tv), l2g2(xsi * e2, xsi * e2 * e3, sv), 1.0);
-        ADD(l2g2(xsi * e2, xsi * e2 * e3, tv), l2g2(xsi, xsi * e1, sv), 1.0);
+        a0 = xsi;
+        if (sub > 0)
+            f = e2;
+        if (sub == 0)
+        {
+            a1 = xsi * e1 * e3;
+            b0 = xsi * (1.0 - e12);
+            b1 = xsi * e1 * (1.0 - e2);
+        }
+        else if (sub == 1)
+        {
+            a1 = xsi * e1;
+            b0 = xsi * (1.0 - e123);
+            b1 = xsi * e1 * e2 * (1 - e3);
+        }
+        else
+        {
+            swap = true;
+            a1 = sub == 2 ? xsi * e123 : sub == 3 ? xsi * e1 : xsi * e12;
+            b0 = sub == 2 ? xsi * (1.0 - e12) : xsi * (1.0 - e123);
+            b1 = sub == 2 ? xsi * e1 * (1.0 - e2) : sub == 3 ? xsi * e12 * (1.0 - e3) : xsi * e1 * (1.0 - e2 * e3);
+        }
     }
     else
-        return {0, 0};
-#undef ADD
-    double f = jw * w;
-    return {rr * f, ri * f};
+    {
+        swap = sub == 1;
+        a0 = xsi;
+        a1 = xsi * e1;
+        b0 = xsi * e2;
+        b1 = xsi * e2 * e3;
+    }
+    ta = swap ? b0 : a0;
+    tb = swap ? b1 : a1;
+    sa = swap ? a0 : b0;
+    sb = swap ? a1 : b1;
 }
 
 __device__ inline int common_vertices(int a0, int a1, int a2, int b0, int b1, int b2)
 {
     return (a0 == b0) + (a0 == b1) + (a0 == b2) + (a1 == b0) + (a1 == b1) + (a1 == b2) + (a2 == b0) + (a2 == b1) +
            (a2 == b2);
-}
-
-// face2FaceIntegrand (integrand.h:228-259); the near-coincidence test stays in FP32. nn =
-// common vertices; SING selects the code path compiled: the singular rules (nn > 0) or the
-// regular 1-point rule (nn == 0), so the regular kernel carries none of the singular code's
-// registers.
-template <bool SING>
-__device__ inline cdbl f2f64(const float *verts, const int *src, const int *trg, int nn, double kr, double ki,
-                             int type, float threshold)
-{
-    const f3 s0 = ld3(verts, src[0]), s1 = ld3(verts, src[1]), s2 = ld3(verts, src[2]);
-    const f3 t0 = ld3(verts, trg[0]), t1 = ld3(verts, trg[1]), t2 = ld3(verts, trg[2]);
-    const float dist = lengthf((s0 + s1 + s2) / 3.0f - (t0 + t1 + t2) / 3.0f);
-    if (dist < threshold && nn == 0)
-        return {0, 0};
-    const TriD S = tri_d(verts, src[0], src[1], src[2]);
-    const TriD T = tri_d(verts, trg[0], trg[1], trg[2]);
-    if constexpr (!SING)
-    {
-        d3 a = l2g(TRI1_X, TRI1_X, S.v), b = l2g(TRI1_X, TRI1_X, T.v);
-        cdbl g = layer64(a, b, S.n, kr, ki, type);
-        double f = 0.25 * TRI1_W * TRI1_W * S.jac * T.jac;
-        return {f * g.re, f * g.im};
-    }
-    else
-    {
-        double rr = 0, ri = 0;
-        for (int a = 0; a < 3; a++)
-            for (int b = 0; b < 3; b++)
-                for (int c = 0; c < 3; c++)
-                    for (int d = 0; d < 3; d++)
-                    {
-                        cdbl p = sing_point64(c_gx[a], c_gx[b], c_gx[c], c_gx[d],
-                                              c_gw[a] * c_gw[b] * c_gw[c] * c_gw[d], S.v, T.v, S.n, nn, kr, ki, type);
-                        rr += p.re;
-                        ri += p.im;
-                    }
-        double f = S.jac * T.jac / 16;
-        return {rr * f, ri * f};
-    }
 }
 
 // Inverse transform with the reference's radix-2 decimation-in-time butterflies
@@ -242,47 +296,12 @@ __device__ inline void quantize_store(const float *s, const float *d, uint32_t *
 __device__ inline int live_count(const int *n_ptr, const int *err) { return *err != 0 ? 0 : *n_ptr; }
 
 // ---------------------------------------------------------------- grid cache
-// Both layer kernels of one (source point, target) pair: they share r and e^{ikr}, so the
-// values are those of two layer64 calls. Split in two so that the target's part is computed once
-// for the 9 wave numbers.
 // orders one wave's LDS writes before its lanes' reads of them
 __device__ inline void wave_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// The wave-number-free part, per (source point, target): r = |trg - src| (0: the target is the
-// source point, both kernels 0), the denominators 4 pi r and 4 pi r^2 r, and (src - trg) . n.
-struct LayerTarget
-{
-    double r, q0, q1, dn;
-};
-__device__ inline LayerTarget layer_target(d3 src, d3 trg, d3 n)
-{
-    const d3 s0 = trg - src;
-    const double r2 = dotd(s0, s0);
-    if (r2 == 0)
-        return {0, 0, 0, 0};
-    const double r = sqrt(r2);
-    const d3 s1 = src - trg;  // = -s0 exactly, so dotd(s1, s1) == r2
-    return {r, 4 * PI_R * r, 4 * PI_R * r2 * r, dotd(s1, n)};
-}
-__device__ inline void layer64_pair(const LayerTarget &t, double kr, double ki, cdbl &g0, cdbl &g1)
-{
-    if (t.r == 0)
-    {
-        g0 = g1 = {0, 0};
-        return;
-    }
-    const double zr = -t.r * ki, zi = t.r * kr;
-    const cdbl e = cexp_d(zr, zi);
-    g0 = {e.re / t.q0, e.im / t.q0};
-    const double ar = -e.re / t.q1, ai = -e.im / t.q1;
-    const double br = 1 - zr, bi = -zi;
-    const double pr = ar * br - ai * bi, pi = ar * bi + ai * br;
-    g1 = {pr * t.dn, pi * t.dn};
 }
 
 // The target cells of one triangle's 27 stencil batches, as offsets from its cell: the
@@ -718,11 +737,36 @@ __global__ __launch_bounds__(256) void k_face_lookup(const TriGeom *__restrict__
         atomicAdd(&tsum[(p & ~63) / SCAN_TILE], (int)__popcll(bal));
 }
 
-// Face-cache integrals (pppm_cache.cu:234-271) per (dirty pair, k <= 8, layer): the
-// face-face integral plus the interpolated far-field representation subtracted for corners
-// farther than 1.5h. Regular pairs (no common vertex) take 16 lanes per item: lane 0
-// evaluates the face-face term, lane 1 + w the far-field term of corner w, and lane 0 adds
-// the corner products in corner order, as potential_integrand does.
+// The interpolated far field that face pair (c, j) subtracts (pppm_cache.cu:234-271): corner w of
+// c's base cell counts if it is farther than 1.5 h from j's centre along an axis. Returns whether
+// it does, with the part of its layer kernels without the wave number and its weight.
+__device__ inline bool far_corner(int w, const TriGeom &gc, const TriGeom &gj, const float *__restrict__ interp_c,
+                                  const WeightArgs &a, d3 pj, d3 nj, LayerTarget &t, double &sc)
+{
+    const double lim = (double)a.h * 1.5;
+    const int x = gc.base3.x + (w >> 2), y = gc.base3.y + ((w >> 1) & 1), z = gc.base3.z + (w & 1);
+    const f3 ctr = cell_center_f(x, y, z, a);
+    if (!((double)fabsf(ctr.x - gj.center.x) > lim || (double)fabsf(ctr.y - gj.center.y) > lim ||
+          (double)fabsf(ctr.z - gj.center.z) > lim))
+        return false;
+    t = layer_target(pj, cell_center_d(x, y, z, a), nj);
+    sc = (double)(-interp_c[w]);
+    return true;
+}
+
+// Face-cache integrals (pppm_cache.cu:234-271) of the dirty pairs, per (wave number k <= 8,
+// layer): the face-face integral plus the interpolated far field of the corners farther than
+// 1.5 h, added in corner order as potential_integrand does (integrand.h:209-222).
+//
+// Regular pairs (no common vertex; face2FaceIntegrand's 1-point rule, integrand.h:228-259, zero
+// for nearly coincident centroids). A wave takes FP = 7 pairs: lane 9 g + t first forms the part
+// without the wave number of term t of pair g (0: the face term, 1 + w: corner w) into LDS, then
+// lane 9 g + k evaluates the pair's nine terms at wave number k in order. Bound by FP64
+// instruction issue (an exponential, a sine and a cosine per term and wave number). With a
+// distance, a square root and four divisions per (term, k, layer) on 16 lanes an item, the
+// 1.4M pairs of a 20480-triangle object in a 128^3 grid took 3.76 ms.
+constexpr int FP = 7;
+constexpr int FWPB = B / WAVE;
 __global__ __launch_bounds__(B) void k_face_regular(const float *__restrict__ verts, const int *__restrict__ tris,
                                                     const TriGeom *__restrict__ geom,
                                                     const int *__restrict__ dirty_pairs, const int *__restrict__ n_ptr,
@@ -730,80 +774,109 @@ __global__ __launch_bounds__(B) void k_face_regular(const float *__restrict__ ve
                                                     const float *__restrict__ interp, WeightArgs a, Tdbem bem,
                                                     cdbl *__restrict__ tmp, const int *__restrict__ err)
 {
-    constexpr int L = 16;
-    const long long lanes = (long long)live_count(n_ptr, err) * 18 * L;
-    // the stride is a multiple of 16, so the 16 lanes of an item stay together
-    for (long long e = (long long)blockIdx.x * B + threadIdx.x; e < lanes; e += (long long)gridDim.x * B)
+    struct Terms
     {
-        const long long i = e / L;
-        const int sub = (int)(e % L);
-        const int d = (int)(i / 18), r = (int)(i % 18), layer = r / 9, k = r % 9;
-        const int p = dirty_pairs[d];
-        const int c = owner[p], j = face_nbr[p];
-        const int src[3] = {tris[3 * j], tris[3 * j + 1], tris[3 * j + 2]};
-        const int trg[3] = {tris[3 * c], tris[3 * c + 1], tris[3 * c + 2]};
-        const int nn = common_vertices(src[0], src[1], src[2], trg[0], trg[1], trg[2]);
-        const bool regular = nn == 0;  // the same for the 16 lanes of the item
-        const double kr = bem.wave_re[k], ki = bem.wave_im[k];
-        double pr = 0, pi = 0;
-        bool far_corner = false;
-        if (regular && sub == 0)
+        LayerTarget t[FP * 9];
+        double sc[FP * 9], f0[FP], f1[FP];  // corner weights; factors of the face and the corner terms
+        unsigned on[FP];                    // terms that count (bit t)
+    };
+    __shared__ Terms lds[FWPB];
+    __shared__ double s_kr[9], s_ki[9];
+    if (threadIdx.x < 9)
+    {
+        s_kr[threadIdx.x] = bem.wave_re[threadIdx.x];
+        s_ki[threadIdx.x] = bem.wave_im[threadIdx.x];
+    }
+    __syncthreads();
+    Terms &T = lds[threadIdx.x >> 6];
+    const int lane = (int)(threadIdx.x & 63), g = lane / 9, r = lane % 9;
+    const int n = live_count(n_ptr, err);
+    const int stride = (int)gridDim.x * FWPB * FP;
+    for (int base = ((int)blockIdx.x * FWPB + (int)(threadIdx.x >> 6)) * FP; base < n; base += stride)
+    {
+        const int d = base + g;
+        bool regular = false, on = false;
+        if (g < FP && d < n)
         {
-            const cdbl v = f2f64<false>(verts, src, trg, nn, kr, ki, layer, bem.threshold);
-            pr = v.re;
-            pi = v.im;
-        }
-        else if (regular && sub <= 8)
-        {
-            const int w = sub - 1;
-            const TriGeom gc = geom[c], gj = geom[j];
-            const double lim = (double)a.h * 1.5;
-            const int x = gc.base3.x + (w >> 2), y = gc.base3.y + ((w >> 1) & 1), z = gc.base3.z + (w & 1);
-            const f3 ctr = cell_center_f(x, y, z, a);
-            if ((double)fabsf(ctr.x - gj.center.x) > lim || (double)fabsf(ctr.y - gj.center.y) > lim ||
-                (double)fabsf(ctr.z - gj.center.z) > lim)
+            const int p = dirty_pairs[d];
+            const int c = owner[p], j = face_nbr[p];
+            const int src[3] = {tris[3 * j], tris[3 * j + 1], tris[3 * j + 2]};
+            const int trg[3] = {tris[3 * c], tris[3 * c + 1], tris[3 * c + 2]};
+            regular = common_vertices(src[0], src[1], src[2], trg[0], trg[1], trg[2]) == 0;
+            if (regular)
             {
                 const TriD J = tri_d(verts, src[0], src[1], src[2]);
                 const d3 pj = l2g(TRI1_X, TRI1_X, J.v);
-                const cdbl g = layer64(pj, cell_center_d(x, y, z, a), J.n, kr, ki, layer);
-                const double sc = (double)(-interp[8 * c + w]);
-                pr = g.re * sc;
-                pi = g.im * sc;
-                far_corner = true;
+                if (r == 0)
+                {
+                    // the near-coincidence test stays in FP32
+                    const f3 s0 = ld3(verts, src[0]), s1 = ld3(verts, src[1]), s2 = ld3(verts, src[2]);
+                    const f3 t0 = ld3(verts, trg[0]), t1 = ld3(verts, trg[1]), t2 = ld3(verts, trg[2]);
+                    on = !(lengthf((s0 + s1 + s2) / 3.0f - (t0 + t1 + t2) / 3.0f) < bem.threshold);
+                    const TriD C = tri_d(verts, trg[0], trg[1], trg[2]);
+                    T.t[lane] = layer_target(pj, l2g(TRI1_X, TRI1_X, C.v), J.n);
+                    T.f0[g] = 0.25 * TRI1_W * TRI1_W * J.jac * C.jac;
+                    T.f1[g] = 0.5 * TRI1_W * J.jac;
+                }
+                else
+                    on = far_corner(r - 1, geom[c], geom[j], interp + 8 * c, a, pj, J.n, T.t[lane], T.sc[lane]);
             }
         }
-        double sr = 0, si = 0;
-        bool any = false;
-#pragma unroll
-        for (int w = 0; w < 8; w++)
+        const unsigned long long mask = __ballot(on);
+        wave_sync();
+        if (regular)
         {
-            const double xr = __shfl(pr, w + 1, L), xi = __shfl(pi, w + 1, L);
-            const bool fw = __shfl(far_corner ? 1 : 0, w + 1, L) != 0;
-            if (fw)
+            const unsigned m = (unsigned)(mask >> (9 * g)) & 511u;
+            const double kr = s_kr[r], ki = s_ki[r];
+            cdbl v0 = {0, 0}, v1 = {0, 0}, g0, g1;
+            if (m & 1u)
             {
-                sr += xr;
-                si += xi;
-                any = true;
+                layer64_pair(T.t[9 * g], kr, ki, g0, g1);
+                const double f = T.f0[g];
+                v0 = {f * g0.re, f * g0.im};
+                v1 = {f * g1.re, f * g1.im};
             }
-        }
-        if (regular && sub == 0)
-        {
-            cdbl v = {pr, pi};
-            if (any)
+            if (m > 1u)
             {
-                const TriD J = tri_d(verts, src[0], src[1], src[2]);
-                const double f = 0.5 * TRI1_W * J.jac;
-                v.re += f * sr;
-                v.im += f * si;
+                double s0r = 0, s0i = 0, s1r = 0, s1i = 0;
+                for (int w = 1; w <= 8; w++)
+                    if (m >> w & 1u)
+                    {
+                        layer64_pair(T.t[9 * g + w], kr, ki, g0, g1);
+                        const double sc = T.sc[9 * g + w];
+                        s0r += g0.re * sc;
+                        s0i += g0.im * sc;
+                        s1r += g1.re * sc;
+                        s1i += g1.im * sc;
+                    }
+                const double f = T.f1[g];
+                v0.re += f * s0r;
+                v0.im += f * s0i;
+                v1.re += f * s1r;
+                v1.im += f * s1i;
             }
-            tmp[i] = v;
+            tmp[(size_t)d * 18 + r] = v0;
+            tmp[(size_t)d * 18 + 9 + r] = v1;
         }
+        wave_sync();
     }
 }
 
-// Singular pairs (common vertices): one thread per (pair, k, layer), the 81-point rules in
-// sequence, then the corner terms.
-__global__ __launch_bounds__(B) void k_face_singular(const float *__restrict__ verts, const int *__restrict__ tris,
+// Singular pairs (common vertices): the 81-point rules (singular_integrand, integrand.h:149-172),
+// a wave per pair. Per run of 21 points the wave's lanes first
+// form the part without the wave number of every (point, region) into LDS, then take the 189
+// (point, k) items, each adding its regions in order for both layers, and then lanes 0..35 add
+// their (layer, re / im, k) series over the points in order: the sums of the point-by-point loop.
+// The far corners follow the same way, 72 (corner, k) items. Bound by FP64 instruction issue
+// (about 39 exponentials with sine and cosine per point, wave number and triangle; the vector
+// units are busy 86 % of the time). A thread per (pair, k, layer) with every distance, root,
+// division and exponential in its own loop, and most lanes of a wave idle beside regular pairs,
+// took 50.4 ms for the 266k singular pairs of a 20480-triangle object; now 4.3 ms (4.5 ms with 27
+// points and three waves per SIMD, 6.1 ms with branches between the polynomial chains).
+constexpr int SQ = 21;  // points at once: 189 of 192 lanes busy in the (point, k) rounds
+constexpr int SR = 3;   // regions at once: 9.8 KB of LDS a wave, four waves per SIMD
+constexpr int SB = 256;
+__global__ __launch_bounds__(SB, 4) void k_face_singular(const float *__restrict__ verts, const int *__restrict__ tris,
                                                       const TriGeom *__restrict__ geom,
                                                       const int *__restrict__ dirty_pairs,
                                                       const int *__restrict__ n_ptr, const int *__restrict__ owner,
@@ -811,48 +884,161 @@ __global__ __launch_bounds__(B) void k_face_singular(const float *__restrict__ v
                                                       const float *__restrict__ interp, WeightArgs a, Tdbem bem,
                                                       cdbl *__restrict__ tmp, const int *__restrict__ err)
 {
-    const long long items = (long long)live_count(n_ptr, err) * 18;
-    for (long long i = (long long)blockIdx.x * B + threadIdx.x; i < items; i += (long long)gridDim.x * B)
+    struct Parts
     {
-        const int d = (int)(i / 18), r = (int)(i % 18), layer = r / 9, k = r % 9;
-        const int p = dirty_pairs[d];
-        const int c = owner[p], j = face_nbr[p];
-        const int src[3] = {tris[3 * j], tris[3 * j + 1], tris[3 * j + 2]};
-        const int trg[3] = {tris[3 * c], tris[3 * c + 1], tris[3 * c + 2]};
-        const int nn = common_vertices(src[0], src[1], src[2], trg[0], trg[1], trg[2]);
-        if (nn == 0)
-            continue;  // k_face_regular computes this pair
-        const double kr = bem.wave_re[k], ki = bem.wave_im[k];
-        cdbl v = f2f64<true>(verts, src, trg, nn, kr, ki, layer, bem.threshold);
-        // the interpolated far field of the corners farther than 1.5h: potential_integrand
-        // (integrand.h:209-222) over the accepted corners in corner order, accumulated on the fly
-        const TriGeom gc = geom[c], gj = geom[j];
-        const double lim = (double)a.h * 1.5;
-        const TriD J = tri_d(verts, src[0], src[1], src[2]);
-        const d3 pj = l2g(TRI1_X, TRI1_X, J.v);
-        double sr = 0, si = 0;
-        bool any = false;
-        for (int w = 0; w < 8; w++)
+        double t[SR][6][SQ];    // (region, LayerTarget member, point)
+        double f[SR][SQ];       // term factor of (region, point); corner weights
+        double jw[SQ];          // point weight times Jacobian
+        double v[4][SQ * 9];    // value of (point, k): layer 0 re, im, layer 1 re, im
+    };
+    __shared__ Parts lds[SB / WAVE];
+    __shared__ double s_kr[9], s_ki[9];
+    if (threadIdx.x < 9)
+    {
+        s_kr[threadIdx.x] = bem.wave_re[threadIdx.x];
+        s_ki[threadIdx.x] = bem.wave_im[threadIdx.x];
+    }
+    __syncthreads();
+    Parts &P = lds[threadIdx.x >> 6];
+    const int lane = (int)(threadIdx.x & 63);
+    const int n = live_count(n_ptr, err);
+    const int waves = (int)gridDim.x * (SB / WAVE);
+    auto put = [&](int sub, int q, const LayerTarget &t) {
+        P.t[sub][0][q] = t.r;
+        P.t[sub][1][q] = t.q0;
+        P.t[sub][2][q] = t.y0;
+        P.t[sub][3][q] = t.q1;
+        P.t[sub][4][q] = t.y1;
+        P.t[sub][5][q] = t.dn;
+    };
+    auto get = [&](int sub, int q) {
+        return LayerTarget{P.t[sub][0][q], P.t[sub][1][q], P.t[sub][2][q],
+                           P.t[sub][3][q], P.t[sub][4][q], P.t[sub][5][q]};
+    };
+    // a wave looks at `run` dirty pairs at once, a lane each, and takes the singular ones in turn
+    const int run = min(WAVE, max(1, n / waves));
+    for (long long base = (long long)((int)blockIdx.x * (SB / WAVE) + (int)(threadIdx.x >> 6)) * run; base < n;
+         base += (long long)waves * run)
+    {
+        int lc = 0, lj = 0, lnn = 0;
+        if (lane < run && base + lane < n)
         {
-            const int x = gc.base3.x + (w >> 2), y = gc.base3.y + ((w >> 1) & 1), z = gc.base3.z + (w & 1);
-            const f3 ctr = cell_center_f(x, y, z, a);
-            if ((double)fabsf(ctr.x - gj.center.x) > lim || (double)fabsf(ctr.y - gj.center.y) > lim ||
-                (double)fabsf(ctr.z - gj.center.z) > lim)
+            const int p = dirty_pairs[base + lane];
+            lc = owner[p];
+            lj = face_nbr[p];
+            lnn = common_vertices(tris[3 * lj], tris[3 * lj + 1], tris[3 * lj + 2], tris[3 * lc], tris[3 * lc + 1],
+                                  tris[3 * lc + 2]);
+        }
+        for (unsigned long long todo = __ballot(lnn != 0); todo; todo &= todo - 1)
+        {
+            const int at = __builtin_ctzll(todo);
+            const int c = __builtin_amdgcn_readlane(lc, at), j = __builtin_amdgcn_readlane(lj, at);
+            const int nn = __builtin_amdgcn_readlane(lnn, at), nsub = sing_regions(nn);
+            const TriD S = tri_d(verts, tris[3 * j], tris[3 * j + 1], tris[3 * j + 2]);
+            const TriD T = tri_d(verts, tris[3 * c], tris[3 * c + 1], tris[3 * c + 2]);
+            const int fld = lane / 9, fk = lane % 9;  // lanes 0..35: the series they add
+            double acc = 0;
+            for (int q0 = 0; q0 < 81 && nsub; q0 += SQ)
             {
-                const cdbl g = layer64(pj, cell_center_d(x, y, z, a), J.n, kr, ki, layer);
-                const double sc = (double)(-interp[8 * c + w]);
-                sr += g.re * sc;
-                si += g.im * sc;
-                any = true;
+                const int nq = min(SQ, 81 - q0);
+                for (int s0 = 0; s0 < nsub; s0 += SR)
+                {
+                    const int ns = min(SR, nsub - s0);
+                    for (int it = lane; it < SQ * ns; it += WAVE)
+                    {
+                        const int sub = it / SQ, q = it % SQ, pt = min(q0 + q, 80);
+                        const int ia = pt / 27, ib = pt / 9 % 3, ic = pt / 3 % 3, id = pt % 3;
+                        const double xsi = 0.5 * (c_gx[ia] + 1), e1 = 0.5 * (c_gx[ib] + 1), e2 = 0.5 * (c_gx[ic] + 1),
+                                     e3 = 0.5 * (c_gx[id] + 1);
+                        double ta, tb, sa, sb, f;
+                        sing_map(nn, s0 + sub, xsi, e1, e2, e3, ta, tb, sa, sb, f);
+                        put(sub, q, layer_target(l2g2(ta, tb, S.v), l2g2(sa, sb, T.v), S.n));
+                        P.f[sub][q] = f;
+                        if (sub == 0)
+                        {
+                            const double w = c_gw[ia] * c_gw[ib] * c_gw[ic] * c_gw[id];
+                            const double jw = nn == 3   ? xsi * xsi * xsi * e1 * e1 * e2
+                                              : nn == 2 ? xsi * xsi * xsi * e1 * e1
+                                                        : xsi * xsi * xsi * e2;
+                            P.jw[q] = jw * w;
+                        }
+                    }
+                    wave_sync();
+                    for (int it = lane; it < nq * 9; it += WAVE)
+                    {
+                        const int q = it / 9, k = it % 9;
+                        const double kr = s_kr[k], ki = s_ki[k];
+                        double r0 = 0, i0 = 0, r1 = 0, i1 = 0;
+                        if (s0 > 0)
+                            r0 = P.v[0][it], i0 = P.v[1][it], r1 = P.v[2][it], i1 = P.v[3][it];
+                        for (int sub = 0; sub < ns; sub++)
+                        {
+                            cdbl g0, g1;
+                            layer64_pair(get(sub, q), kr, ki, g0, g1);
+                            const double f = P.f[sub][q];
+                            r0 += g0.re * f;
+                            i0 += g0.im * f;
+                            r1 += g1.re * f;
+                            i1 += g1.im * f;
+                        }
+                        const double f = s0 + SR < nsub ? 1.0 : P.jw[q];  // (after the last region)
+                        P.v[0][it] = r0 * f;
+                        P.v[1][it] = i0 * f;
+                        P.v[2][it] = r1 * f;
+                        P.v[3][it] = i1 * f;
+                    }
+                    wave_sync();
+                }
+                if (lane < 36)
+                {
+#pragma unroll 3
+                    for (int q = 0; q < nq; q++)  // nq is a multiple of 3
+                        acc += P.v[fld][9 * q + fk];
+                }
+                wave_sync();
             }
+            // the interpolated far field of the far corners
+            bool on = false;
+            if (lane < 8)
+            {
+                LayerTarget t{};
+                double sc = 0;
+                on = far_corner(lane, geom[c], geom[j], interp + 8 * c, a, l2g(TRI1_X, TRI1_X, S.v), S.n, t, sc);
+                put(0, lane, t);
+                P.f[0][lane] = sc;
+            }
+            const unsigned far = (unsigned)(__ballot(on) & 255u);
+            wave_sync();
+            if (far)
+                for (int it = lane; it < 72; it += WAVE)
+                {
+                    const int w = it / 9, k = it % 9;
+                    cdbl g0 = {0, 0}, g1 = {0, 0};
+                    if (far >> w & 1u)
+                        layer64_pair(get(0, w), s_kr[k], s_ki[k], g0, g1);
+                    const double sc = P.f[0][w];
+                    P.v[0][it] = g0.re * sc;
+                    P.v[1][it] = g0.im * sc;
+                    P.v[2][it] = g1.re * sc;
+                    P.v[3][it] = g1.im * sc;
+                }
+            wave_sync();
+            if (lane < 36)
+            {
+                double v = acc * (S.jac * T.jac / 16);
+                if (far)
+                {
+                    double s = 0;
+                    for (int w = 0; w < 8; w++)
+                        if (far >> w & 1u)
+                            s += P.v[fld][9 * w + fk];
+                    v += 0.5 * TRI1_W * S.jac * s;
+                }
+                double *out = reinterpret_cast<double *>(tmp + (size_t)(base + at) * 18 + (fld >> 1) * 9 + fk);
+                out[fld & 1] = v;
+            }
+            wave_sync();
         }
-        if (any)
-        {
-            const double f = 0.5 * TRI1_W * J.jac;
-            v.re += f * sr;
-            v.im += f * si;
-        }
-        tmp[i] = v;
     }
 }
 
@@ -993,10 +1179,11 @@ hipError_t launch_face_weights(const float *verts, const int *tris, const TriGeo
                                float2 *fsc, float2 *fmeta, const int *err, long long hint_dirty, hipStream_t s)
 {
     const long long hint = hint_dirty < 0 ? cap : std::min<long long>(hint_dirty, cap);
-    k_face_regular<<<nb_hint(hint * 18 * 16, (long long)cap * 18 * 16, B), B, 0, s>>>(
-        verts, tris, geom, dirty_pairs, n_ptr, owner, face_nbr, interp, a, b, (cdbl *)tmp, err);
-    k_face_singular<<<nb_hint(hint * 18, (long long)cap * 18, B), B, 0, s>>>(
-        verts, tris, geom, dirty_pairs, n_ptr, owner, face_nbr, interp, a, b, (cdbl *)tmp, err);
+    k_face_regular<<<nb_hint(hint, cap, FWPB * FP), B, 0, s>>>(verts, tris, geom, dirty_pairs, n_ptr, owner, face_nbr,
+                                                              interp, a, b, (cdbl *)tmp, err);
+    // a wave per dirty pair, or per run of them where the launch's cap is reached
+    k_face_singular<<<nb_hint(hint, cap, SB / WAVE), SB, 0, s>>>(verts, tris, geom, dirty_pairs, n_ptr, owner, face_nbr,
+                                                                interp, a, b, (cdbl *)tmp, err);
     k_face_finish<<<nb_hint(hint, cap, B), B, 0, s>>>(dirty_pairs, n_ptr, face_slot, geom, owner, face_nbr, b,
                                                   (const cdbl *)tmp, fw, fsc, fmeta, err);
     return hipGetLastError();
