@@ -334,6 +334,18 @@ int pppm_batch_run(pppm_batch *b, const float *const *neumann_series, const long
                                   out_dev + (size_t)i * n_listen);
         hd[i].out_stride = (long long)n * n_listen;
     }
+    // the waves of a launch are those of all scenes together
+    long long w3 = 0, w4 = 0;
+    for (const SceneStep &d : hd)
+    {
+        w3 += d.c3_waves;
+        w4 += d.face_waves;
+    }
+    for (SceneStep &d : hd)
+    {
+        d.gran3 = gather_gran(w3);
+        d.gran4 = gather_gran(w4);
+    }
     BCK(b->descs.ensure(n));
     BCK(hipMemcpyAsync(b->descs.p, hd.data(), n * sizeof(SceneStep), hipMemcpyHostToDevice, b->stream));
     std::vector<int> nw(n), nf(n), nd(n), nn(n);

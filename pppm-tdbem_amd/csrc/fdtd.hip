@@ -360,13 +360,13 @@ __global__ __launch_bounds__(BLK) void k_fdtd_abc(float *__restrict__ grid3, Fdt
         fdtd_block(grid3, p, t, blk, nb_inner);
     else
     {
-        // windows for the step that follows (t + 1): row k < 15 = ring value at t - k, row 15 =
-        // ring slot t + 1 (overwritten by the far-field and Dirichlet launches before use)
+        // windows for the step that follows (t + 1): row k = ring value at t + 1 - k (row 0 is
+        // overwritten by the far-field and Dirichlet launches before use)
         const int i = (blk - nb_fdtd) * BLK + (int)threadIdx.x;
         if (i < f.nt * STEPS)
         {
             const int tri = i / STEPS, k = i % STEPS;
-            const int slot = (k == STEPS - 1 ? t + 1 : t - k) & (RING - 1);
+            const int slot = (t + 1 - k) & (RING - 1);
             f.wn[i] = f.hn[tri * RING + slot];
             f.wd[i] = f.hd[tri * RING + slot];
         }

@@ -330,6 +330,8 @@ struct SceneStep
     int c3_waves;
     // face gather (Dirichlet update)
     int face_waves;
+    // wave-map entries (64 pairs each) a wave of the C3 gathers / the face gather takes
+    int gran3, gran4;
     const int *face_start, *face_wave, *face_nbr, *face_slot;
     const uint32_t *wf, *wb, *fw;  // 16 x half2 {S_k, D_k} per record
     const float2 *sf, *sb, *fsc;   // scales
@@ -351,8 +353,17 @@ struct SceneStep
     float *out;
     long long out_stride;
 };
-// history windows of the gathers: wn/wd[tri*16 + k] = ring value at t - back - k, with t the
-// device time index when the kernel runs (back = 0 before the advance of a step, 1 after)
+// Wave-map entries (64 pairs each) per wave of a gather whose maps hold `waves` entries (all
+// scenes of a launch together). A wave spends about as long on its start (map, descriptor, first
+// indices) and on its segments' ends as on a round of 64 pairs, so where there are waves enough to
+// fill the device several times each takes up to four entries, and where there are few, one.
+// Measured per step, 1 / 2 / 4 entries: 32^3 / 1280 triangles (1.5k entries) 21 / 24 / 31 us alone;
+// 141^3 / 20480 triangles (22k face entries) 2.71 / 2.51 / 2.58 ms for 32 steps; 64 scenes (111k
+// face, 42k C3 entries) 18.2 / 16.4 / 16.0 ms for 32 steps.
+constexpr int gather_gran(long long waves) { return waves >= 4 * 8192 ? 4 : waves >= 2 * 8192 ? 2 : 1; }
+// history windows of the gathers: wn/wd[tri*16 + k] = ring value of time t - k, the value of tap k
+// (t: the step the gathers serve, the device time index plus 1 - back when the kernel runs: back =
+// 0 before the advance of a step, 1 after)
 hipError_t launch_windows(const SceneStep &d, int back, hipStream_t s);
 hipError_t launch_far(const SceneStep &d, hipStream_t s);
 hipError_t launch_dirichlet(const SceneStep &d, hipStream_t s);

@@ -601,6 +601,8 @@ SceneStep scene_step(const pppm_solver *s, const StepBufs &b, const float *neuma
     d.c3_pairs = s->c3_pairs.p;
     d.c3_waves = s->c3_waves;
     d.face_waves = s->face_waves;
+    d.gran3 = gather_gran(s->c3_waves);
+    d.gran4 = gather_gran(s->face_waves);
     d.face_start = s->face_start.p;
     d.face_wave = s->face_wave.p;
     d.face_nbr = s->face_nbr.p;

@@ -7,20 +7,27 @@
 // solve_fdtd_near_kernel (pppm.cu:53-114), LayerWeightHalf::convolution (bem.h:203-213).
 //
 // Segmented gather with a fixed summation order. A "segment" is a C3 cell (far / near)
-// or a triangle (Dirichlet); its pairs are contiguous in a CSR list. Wave w owns the
-// segments whose first pair lies in [64w, 64w+64) — at most 64, one leader lane each;
-// the owned range comes from a wave map built with the lists, which also holds the first
-// pair of that range, so a wave starts with two 8-byte loads. The wave walks its pair
-// range in rounds of 64: lane i evaluates the 16-tap convolution of pair (round base + i)
-// sequentially (k = 0..15, as the reference's loop), parks the value in LDS, and every
-// leader adds the values of its own pairs in list order. Every sum therefore has the
-// order of a sequential loop, whatever the segment lengths, and lanes stay busy across
-// segment boundaries.
+// or a triangle (Dirichlet); its pairs are contiguous in a CSR list. Entry w of the wave map
+// built with the lists holds the segments whose first pair lies in [64w, 64w+64) and the first
+// pair of that range; a wave takes one, two or four entries (gather_gran) and walks their pairs
+// in rounds of 64. Four lanes fetch a pair's record and windows and form its 16 terms, the pair's
+// lane adds them sequentially (k = 0..15, as the reference's loop) and parks the value in LDS;
+// after a chunk of 256 pairs each lane adds the values of its own segment in list order
+// (gather_wave). Every sum therefore has the order of a sequential loop, whatever the segment
+// lengths, and lanes stay busy across segment boundaries.
+//
+// What bounds it: the records' HBM stream (without it the far and near gathers of 64 scenes take
+// half the time), then the waves' serial start and end. One lane fetching its pair's 64 B rows
+// and every lane sweeping all 64 values of a round for its sums issued 620 vector instructions
+// and 500 cache accesses per round; now about 230 and 190. 64 scenes together (7.45M face, 2.68M
+// cell pairs): Dirichlet 181 -> 166 us, near 99 -> 72 us, far 87 -> 73 us. Fetching a round's
+// records one round ahead, or all of a round's loads at once, costs two waves per SIMD and was
+// slower (187, 175 us Dirichlet).
 //
 // Weights: 64 B record per pair (16 x half2 {S_k, D_k}) + float2 scales. History: the
 // reference's 32-slot rings (slot = t mod 32), one 128 B line per triangle and field, plus
-// per-step windows of the 16 latest values in time order (one 64 B row per triangle and
-// field) from which the gathers read taps 1..15 as four 16 B loads.
+// per-step windows of the 16 latest values in tap order (one 64 B row per triangle and field)
+// from which the gathers read.
 //
 // Time index: all kernels read t from device memory (StepState), so one captured HIP
 // graph replays any step.
@@ -50,101 +57,206 @@ __device__ inline void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// acc plus the values vals[lo], ..., vals[hi - 1] of one round (64 values parked by the wave's
-// lanes, 16-byte aligned), added one at a time in that order: the sequential loop's sum. Every
-// lane sweeps all 64 positions with 16-byte LDS reads (the same addresses in every lane, so
-// broadcasts) and keeps acc where a position is outside its range, so a round costs four
-// waits on LDS instead of one per value, and lanes with several short ranges (or none) run
-// in step. Positions outside [lo, hi) leave acc bit for bit as it was (a select, not + 0).
-__device__ __forceinline__ float round_sum(float acc, const float *__restrict__ vals, int lo, int hi)
+// Pairs a wave convolves and parks in LDS before its lanes add them up: enough that the segments
+// of a chunk are many and most rounds of 64 full.
+constexpr int CH = 4 * WAVE;
+
+// LDS of one wave of a gather: the terms of a round, the values of a chunk
+template <class V>
+struct GatherLds
 {
-    if (lo <= 0 && hi >= WAVE)
-    {
-        // the whole round belongs to this lane's segment (the usual case of the long face lists)
+    float4 term[4 * WAVE];
+    V vals[CH];
+};
+
+// acc plus vals[0], ..., vals[n - 1], added one at a time in that order (V: float, or float2
+// for two sums side by side). Each lane reads its own range: sixteen at a time, then the rest
+// by halves, so the wave issues about as many additions as its longest segment has values.
+template <int K, class V>
+__device__ __forceinline__ void add_run(V &acc, const V *&vals)
+{
+    V v[K];
 #pragma unroll
-        for (int c = 0; c < WAVE; c += 16)
-        {
-            float v[16];
+    for (int i = 0; i < K; i++)
+        v[i] = vals[i];
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-                *reinterpret_cast<float4 *>(&v[4 * i]) = reinterpret_cast<const float4 *>(vals + c)[i];
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-                acc += v[i];
-        }
-        return acc;
-    }
-    if (lo >= hi)
-        return acc;
-#pragma unroll
-    for (int c = 0; c < WAVE; c += 16)
-    {
-        float v[16];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            *reinterpret_cast<float4 *>(&v[4 * i]) = reinterpret_cast<const float4 *>(vals + c)[i];
-#pragma unroll
-        for (int i = 0; i < 16; i++)
-        {
-            const float sum = acc + v[i];
-            acc = (c + i >= lo && c + i < hi) ? sum : acc;
-        }
-    }
+    for (int i = 0; i < K; i++)
+        acc += v[i];
+    vals += K;
+}
+template <class V>
+__device__ __forceinline__ V segment_sum(V acc, const V *vals, int n)
+{
+    for (; n >= 16; n -= 16)
+        add_run<16>(acc, vals);
+    if (n & 8)
+        add_run<8>(acc, vals);
+    if (n & 4)
+        add_run<4>(acc, vals);
+    if (n & 2)
+        add_run<2>(acc, vals);
+    if (n & 1)
+        add_run<1>(acc, vals);
     return acc;
 }
 
-// LayerWeightHalf::convolution (bem.h:203-213) for one pair, taps K0..15 in order, from the
-// pair triangle's history windows (four 16 B loads per field): rows 0..14 hold the values at
-// t-1 .. t-15 (taps 1..15), row 15 the value at t (tap 0; written into the window by the kernel
-// that produces it, see windows_item). DZERO0: the Dirichlet value of step t is read as 0
-// (pppm.cu:143).
-template <int K0, bool DZERO0>
-__device__ inline float conv_pair(const uint32_t *__restrict__ w16, float2 sc, const float *__restrict__ wn,
-                                  const float *__restrict__ wd, uint32_t *tap0 = nullptr)
+__device__ inline float read_lane(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
+__device__ inline float2 read_lane(float2 v, int l) { return make_float2(read_lane(v.x, l), read_lane(v.y, l)); }
+
+// The segmented gather of one wave over the segments [w0.x, w1.x) and their pairs [w0.y, w1.y):
+// chunks of CH pairs are convolved 64 at a time into LDS (g.load: a pair's indices; g.conv: a round); then lane l adds the
+// part of segment cs + l that lies in the chunk, in list order, and finished segments are handed
+// to g.done. At most one segment is open at a chunk's end; its sum is carried to the next chunk.
+// g.early / g.late load what done needs, behind the first and the last round of a chunk.
+template <class V, class G>
+__device__ __forceinline__ void gather_wave(G &g, const int *__restrict__ start, int2 w0, int2 w1, int lane,
+                                            GatherLds<V> &lds)
 {
-    uint4 q[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        q[i] = reinterpret_cast<const uint4 *>(w16)[i];
-    float4 hn4[4], hd4[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
+    V *__restrict__ vals = lds.vals;
+    int cs = w0.x;
+    const int c1 = w1.x, q0 = w0.y, q1 = w1.y;
+    V carry{};
+    typename G::Index idx = g.load(min(q0 + lane, q1 - 1));
+    for (int base = q0; base < q1; base += CH)
     {
-        hn4[i] = reinterpret_cast<const float4 *>(wn)[i];
-        hd4[i] = reinterpret_cast<const float4 *>(wd)[i];
+        const int end = min(base + CH, q1);
+        int s = cs + lane;
+        int m0 = s < c1 ? start[s] : q1, m1 = s < c1 ? start[s + 1] : q1 + 1;
+        for (int b = base; b < end; b += WAVE)
+        {
+            // the next round's indices are loaded beside this round's records
+            const typename G::Index next = g.load(min(b + WAVE + lane, q1 - 1));
+            g.conv(idx, end - b, lane, lds.term, vals + (b - base));
+            idx = next;
+            if (b == base)
+                g.early(s, s < c1 && (m0 < end || end == q1));
+        }
+        g.late();
+        wave_sync();
+        for (;;)
+        {
+            const bool in = s < c1 && (m0 < end || end == q1), fin = in && m1 <= end;
+            V acc{};
+            if (lane == 0)
+                acc = carry;
+            if (in)
+            {
+                const int lo = max(m0, base);
+                acc = segment_sum(acc, vals + (lo - base), min(m1, end) - lo);
+            }
+            if (fin)
+                g.done(s, acc);
+            const unsigned long long done = __ballot(fin);
+            const int nd = (int)__popcll(done);
+            carry = V{};
+            if (__ballot(in) != done)
+                carry = read_lane(acc, nd);  // finished segments are lanes 0 .. nd - 1
+            cs += nd;
+            if (nd < WAVE || cs >= c1)
+                break;
+            s = cs + lane;
+            m0 = s < c1 ? start[s] : q1;
+            m1 = s < c1 ? start[s + 1] : q1 + 1;
+            g.early(s, s < c1 && (m0 < end || end == q1));
+            g.late();
+        }
+        wave_sync();
     }
-    const uint32_t *w = reinterpret_cast<const uint32_t *>(q);
-    const float *hnw = reinterpret_cast<const float *>(hn4);
-    const float *hdw = reinterpret_cast<const float *>(hd4);
-    if (tap0)
-        *tap0 = w[0];
+}
+
+// map entries [gran * wave, gran * (wave + 1)) of a gather's wave map: its first segment and pair
+__device__ __forceinline__ void wave_range(const int *__restrict__ map, int waves, int gran, int wave, int2 &w0, int2 &w1)
+{
+    w0 = reinterpret_cast<const int2 *>(map)[gran * wave];
+    w1 = reinterpret_cast<const int2 *>(map)[min(gran * (wave + 1), waves)];
+}
+__host__ __device__ inline int gran_waves(int waves, int gran) { return (waves + gran - 1) / gran; }
+
+// LayerWeightHalf::convolution (bem.h:203-213) of a round of up to 64 pairs, taps in order, from the
+// pair triangles' history windows (row k of a window: the value at t - k, tap k). rec / tri: this
+// lane's pair's record and triangle (any valid ones past the round's n pairs). K0: first tap that
+// counts. DZERO0: the Dirichlet value of step t is read as 0 (pppm.cu:143). fac (may be null):
+// receives D_0 times its scale for pair i at fac[2 * i].
+//
+// Four lanes share a pair: lane 4 h + q fetches quarter q of the 64 B record and of both windows
+// of pairs h, 16 + h, 32 + h and 48 + h, so a load instruction covers whole cache lines (1 KB of
+// consecutive records) instead of 16 B of each of 64 rows, and forms the terms of its four taps.
+// They pass through LDS to the lane of the pair, which adds all sixteen in order; quarters are
+// stored at q ^ (pair / 4 mod 4), which keeps both sides free of bank conflicts.
+template <int K0, bool DZERO0>
+__device__ __forceinline__ float conv_round(const uint32_t *__restrict__ w16, const float2 *__restrict__ scale, int rec,
+                                            int tri, int n, const float *__restrict__ wn, const float *__restrict__ wd,
+                                            int lane, float4 *__restrict__ term, float *__restrict__ fac)
+{
+    const int h = lane >> 2, q = lane & 3;
+    const int col = q ^ ((h >> 2) & 3);
+    wave_sync();  // the reads of the round before
+#pragma unroll
+    for (int half = 0; half < 2; half++)
+    {
+        if (32 * half >= n)
+            break;
+        uint4 w[2];
+        float4 hn[2], hd[2];
+        float2 sc[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+        {
+            const int src = 32 * half + 16 * i + h;
+            const int r = __shfl(rec, src), t = __shfl(tri, src);
+            w[i] = reinterpret_cast<const uint4 *>(w16)[4 * (size_t)r + q];
+            sc[i] = scale[r];
+            hn[i] = reinterpret_cast<const float4 *>(wn)[4 * (size_t)t + q];
+            hd[i] = reinterpret_cast<const float4 *>(wd)[4 * (size_t)t + q];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+        {
+            const int pair = 32 * half + 16 * i + h;
+            if (DZERO0 && q == 0)
+                hd[i].x = 0.0f;
+            const uint32_t ww[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+            const float nn[4] = {hn[i].x, hn[i].y, hn[i].z, hn[i].w}, dd[4] = {hd[i].x, hd[i].y, hd[i].z, hd[i].w};
+            float v[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+            {
+                const float a = -f16_bits_to_f32(ww[c]) * sc[i].x * nn[c];
+                const float b = f16_bits_to_f32(ww[c] >> 16) * sc[i].y * dd[c];
+                v[c] = a + b;
+            }
+            term[4 * pair + col] = make_float4(v[0], v[1], v[2], v[3]);
+            if (fac && q == 0)
+                fac[2 * pair] = f16_bits_to_f32(ww[0] >> 16) * sc[i].y;
+        }
+    }
+    wave_sync();
     float r = 0.0f;
 #pragma unroll
-    for (int k = K0; k < STEPS; k++)
+    for (int qq = 0; qq < 4; qq++)
     {
-        const float ws = f16_bits_to_f32(w[k]);
-        const float wdk = f16_bits_to_f32(w[k] >> 16);
-        const float n = k == 0 ? hnw[STEPS - 1] : hnw[k - 1];
-        const float d = k == 0 ? (DZERO0 ? 0.0f : hdw[STEPS - 1]) : hdw[k - 1];
-        const float a = -ws * sc.x * n;
-        const float b = wdk * sc.y * d;
-        r += a + b;
+        const float4 v = term[4 * lane + (qq ^ ((lane >> 2) & 3))];
+        if (qq > 0 || K0 == 0)
+            r += v.x;
+        r += v.y;
+        r += v.z;
+        r += v.w;
     }
     return r;
 }
 
-// History windows for the gathers of step t: row k < 15 of triangle i holds the ring value at
-// t - 1 - k, so a gather reads tap k >= 1 at row k - 1; row 15 holds the value at t (tap 0).
-// back = 0 when launched before t is advanced (the time step: the values at t do not exist yet;
-// the far-field launch writes the Neumann value and the Dirichlet update the Dirichlet value
-// into row 15 as into the ring), 1 after it (the phase entry points: the ring holds them).
+// History windows for the gathers of step t: row k of triangle i holds the ring value at t - k, the
+// value of tap k. back = 0 when launched before t is advanced (the time step: the values at t do
+// not exist yet; the far-field launch writes the Neumann value and the Dirichlet update the
+// Dirichlet value into row 0 as into the ring), 1 after it (the phase entry points: the ring
+// holds them).
 __device__ __forceinline__ void windows_item(const SceneStep &d, int back, int i)
 {
     if (i >= d.a.nt * STEPS || (d.err && *d.err))
         return;
     const int tri = i / STEPS, k = i % STEPS;
     const int tn = d.st->t - back + 1;  // t of the step the gathers serve
-    const int slot = (k == STEPS - 1 ? tn : tn - 1 - k) & (RING - 1);
+    const int slot = (tn - k) & (RING - 1);
     d.wn[i] = d.hn[tri * RING + slot];
     d.wd[i] = d.hd[tri * RING + slot];
 }
@@ -152,65 +264,55 @@ __device__ __forceinline__ void windows_item(const SceneStep &d, int back, int i
 // far(c) = p(c) - sum_pairs W^fdtd (*) (N, D). W^fdtd has tap 0 == 0 (pppm_cache.cu:111),
 // so taps 1..15 only (adding the zero tap leaves the sum bit-identical); the Neumann slot
 // of step t is therefore free to be written by the extra waves of this launch.
-__device__ __forceinline__ void far_wave(const SceneStep &d, int wave, int lane, float *__restrict__ vals)
+struct FarGather
+{
+    struct Index
+    {
+        int p, rec;
+    };
+    const SceneStep &d;
+    const float *g;
+    size_t nn;
+    unsigned cell;
+    float gv;
+    __device__ __forceinline__ Index load(int p) const { return Index{p, d.c3_pairs[p]}; }
+    __device__ __forceinline__ void conv(Index i, int n, int lane, float4 *term, float *vals) const
+    {
+        vals[lane] = conv_round<1, false>(d.owf ? d.owf : d.wf, d.owf ? d.osf : d.sf, d.owf ? i.p : i.rec, i.rec / GC, n,
+                                          d.wn, d.wd, lane, term, nullptr);
+    }
+    __device__ __forceinline__ void early(int s, bool in) { cell = in ? (unsigned)d.c3_cells[s] : ~0u; }
+    __device__ __forceinline__ void late() { gv = cell < nn ? g[cell] : 0.0f; }
+    __device__ __forceinline__ void done(int s, float acc) const { d.far[s] = cell < nn ? gv - acc : 0.0f; }
+};
+__device__ __forceinline__ void far_wave(const SceneStep &d, int wave, int lane, GatherLds<float> &lds)
 {
     // the wave map is read before the error word is waited on (in bounds either way), so the
     // two loads take one memory round trip
+    const int nw = gran_waves(d.c3_waves, d.gran3);
     int2 w0 = {0, 0}, w1 = {0, 0};
-    if (wave < d.c3_waves)
-    {
-        w0 = reinterpret_cast<const int2 *>(d.c3_wave)[wave];
-        w1 = reinterpret_cast<const int2 *>(d.c3_wave)[wave + 1];
-    }
+    if (wave < nw)
+        wave_range(d.c3_wave, d.c3_waves, d.gran3, wave, w0, w1);
     if (d.err && *d.err)  // behind a mesh update that failed: the step is run again after the update is
         return;
     const int t = d.st->t;
-    if (wave < d.c3_waves)
+    if (wave < nw)
     {
-        const int c0 = w0.x, q0 = w0.y, c1 = w1.x, q1 = w1.y;
-        if (c0 >= c1)
+        if (w0.x >= w1.x)
             return;
         const size_t nn = (size_t)d.a.N * d.a.N * d.a.N;
-        const float *g = d.grid3 + (size_t)(((t % 3) + 3) % 3) * nn;
-        const int cs = c0 + lane;
-        const bool leader = cs < c1;
-        // every index of the wave's first round is loaded at once, then what they point to
-        const int m0 = leader ? d.c3_start[cs] : 0, m1 = leader ? d.c3_start[cs + 1] : 0;
-        const unsigned cell = leader ? (unsigned)d.c3_cells[cs] : ~0u;
-        int rec = q0 + lane < q1 ? d.c3_pairs[q0 + lane] : -1;
-        const float gv = cell < nn ? g[cell] : 0.0f;
-        float acc = 0.0f;
-        for (int base = q0; base < q1; base += WAVE)
-        {
-            const int p = base + lane;
-            // the next round's index is loaded now, beside this round's records
-            const int rec_next = p + WAVE < q1 ? d.c3_pairs[p + WAVE] : -1;
-            float v = 0.0f;
-            if (p < q1)  // rec >= 0 exactly then; the list-ordered record does not wait for rec
-            {
-                const int tri = rec / GC;
-                const uint32_t *w = d.owf ? d.owf + (size_t)p * STEPS : d.wf + (size_t)rec * STEPS;
-                const float2 sc = d.owf ? d.osf[p] : d.sf[rec];
-                v = conv_pair<1, false>(w, sc, d.wn + tri * STEPS, d.wd + tri * STEPS);
-            }
-            vals[lane] = v;
-            wave_sync();
-            acc = round_sum(acc, vals, max(m0, base) - base, min(m1, base + WAVE) - base);
-            wave_sync();
-            rec = rec_next;
-        }
-        if (leader)
-            d.far[cs] = cell < nn ? gv - acc : 0.0f;
+        FarGather g{d, d.grid3 + (size_t)(((t % 3) + 3) % 3) * nn, nn, ~0u, 0.0f};
+        gather_wave(g, d.c3_start, w0, w1, lane, lds);
     }
     else
     {
         // Neumann input of step t into the ring (set_neumann_condition_kernel)
-        const int i = (wave - d.c3_waves) * WAVE + lane;
+        const int i = (wave - nw) * WAVE + lane;
         if (d.neumann && i < d.a.nt)
         {
             const float v = d.neumann[(size_t)(t - d.a.t0) * d.a.stride + i];
             d.hn[i * RING + (t & (RING - 1))] = v;
-            d.wn[i * STEPS + STEPS - 1] = v;  // tap 0 of the Dirichlet update and the near field
+            d.wn[i * STEPS] = v;  // tap 0 of the Dirichlet update and the near field
         }
     }
 }
@@ -218,102 +320,113 @@ __device__ __forceinline__ void far_wave(const SceneStep &d, int wave, int lane,
 // Face far field (8-corner interpolation, pppm.cu:116-144), face near field against the
 // 4x4x4 list with D[t] = 0 and its tap-0 factors (pppm.cu:146-170), then
 // D_c[t] = (far*rc + near) / (0.5*area - sum_j D_0(c, j)) (pppm.cu:172-193).
-__device__ __forceinline__ void dirichlet_wave(const SceneStep &d, int wave, int lane, float *__restrict__ vals,
-                                               float *__restrict__ facs)
+// The two sums of a pair are parked side by side: x the convolution, y the tap-0 factor.
+struct FaceGather
 {
-    const int t = d.st->t;
-    if (wave >= d.face_waves)
-        return;
-    // the wave map is read before the error word is waited on (one memory round trip)
-    const int2 w0 = reinterpret_cast<const int2 *>(d.face_wave)[wave];
-    const int2 w1 = reinterpret_cast<const int2 *>(d.face_wave)[wave + 1];
-    // after a flagged mesh update the face lists may be incomplete: leave D[t] untouched
-    if (*d.err != 0)
-        return;
-    const int c0 = w0.x, q0 = w0.y, c1 = w1.x, q1 = w1.y;
-    if (c0 >= c1)
-        return;
-    const int cs = c0 + lane;
-    const bool leader = cs < c1;
-    // every index of the wave's first round is loaded at once, then what they point to; the
-    // leaders' face far field (8-corner interpolation) does not depend on the gather
-    const int m0 = leader ? d.face_start[cs] : 0, m1 = leader ? d.face_start[cs + 1] : 0;
-    int j = -1, ws = 0;
-    if (q0 + lane < q1)
+    struct Index
     {
-        j = d.face_nbr[q0 + lane];
-        ws = d.face_slot[q0 + lane];
+        int j, rec;
+    };
+    const SceneStep &d;
+    int t;
+    int s;  // this lane's segment of the chunk, -1: none
+    float ff, area;
+    __device__ __forceinline__ Index load(int p) const { return Index{d.face_nbr[p], d.ofw ? p : d.face_slot[p]}; }
+    __device__ __forceinline__ void conv(Index i, int n, int lane, float4 *term, float2 *vals) const
+    {
+        vals[lane].x = conv_round<0, true>(d.ofw ? d.ofw : d.fw, d.ofw ? d.ofsc : d.fsc, i.rec, i.j, n, d.wn, d.wd, lane,
+                                           term, &vals[0].y);  // face_factor = (float)D_0 * scale_D
     }
-    float ff = 0.0f, area = 0.0f;
-    if (leader)
+    __device__ __forceinline__ void early(int s_, bool in) { s = in ? s_ : -1; }
+    __device__ __forceinline__ void late()
     {
+        if (s < 0)
+            return;
         int ci[8];
         float iw[8];
 #pragma unroll
         for (int w = 0; w < 8; w++)
         {
-            ci[w] = d.corner[8 * cs + w];  // corners of a base cell are C3 cells (>= 0)
-            iw[w] = d.interp[8 * cs + w];
+            ci[w] = d.corner[8 * s + w];  // corners of a base cell are C3 cells (>= 0)
+            iw[w] = d.interp[8 * s + w];
         }
-        area = d.geom[cs].area;
+        area = d.geom[s].area;
+        ff = 0.0f;
 #pragma unroll
         for (int w = 0; w < 8; w++)
             ff += iw[w] * (ci[w] >= 0 ? d.far[ci[w]] : 0.0f);
     }
-    float acc = 0.0f, fac = 0.0f;
-    for (int base = q0; base < q1; base += WAVE)
+    __device__ __forceinline__ void done(int s, float2 acc) const
     {
-        const int p = base + lane;
-        // the next round's indices are loaded now, beside this round's records
-        int j_next = -1, ws_next = 0;
-        if (p + WAVE < q1)
-        {
-            j_next = d.face_nbr[p + WAVE];
-            ws_next = d.face_slot[p + WAVE];
-        }
-        float v = 0.0f, f = 0.0f;
-        if (p < q1)  // j >= 0 exactly then; the list-ordered record does not wait for the slot
-        {
-            const float2 sc = d.ofw ? d.ofsc[p] : d.fsc[ws];
-            const uint32_t *w = d.ofw ? d.ofw + (size_t)p * STEPS : d.fw + (size_t)ws * STEPS;
-            uint32_t tap0;
-            v = conv_pair<0, true>(w, sc, d.wn + j * STEPS, d.wd + j * STEPS, &tap0);
-            f = f16_bits_to_f32(tap0 >> 16) * sc.y;  // face_factor = (float)D_0 * scale_D
-        }
-        vals[lane] = v;
-        facs[lane] = f;
-        wave_sync();
-        {
-            const int lo = max(m0, base) - base, hi = min(m1, base + WAVE) - base;
-            acc = round_sum(acc, vals, lo, hi);
-            fac = round_sum(fac, facs, lo, hi);
-        }
-        wave_sync();
-        j = j_next;
-        ws = ws_next;
-    }
-    if (leader)
-    {
-        const float num = ff * d.a.rc + acc;
-        const double den = 0.5 * (double)area - (double)fac;
+        const float num = ff * d.a.rc + acc.x;
+        const double den = 0.5 * (double)area - (double)acc.y;
         const float dv = (float)((double)num / den);
-        d.hd[cs * RING + (t & (RING - 1))] = dv;
-        d.wd[cs * STEPS + STEPS - 1] = dv;  // tap 0 of the near field
+        d.hd[s * RING + (t & (RING - 1))] = dv;
+        d.wd[s * STEPS] = dv;  // tap 0 of the near field
     }
+};
+__device__ __forceinline__ void dirichlet_wave(const SceneStep &d, int wave, int lane, GatherLds<float2> &lds)
+{
+    const int t = d.st->t;
+    if (wave >= gran_waves(d.face_waves, d.gran4))
+        return;
+    // the wave map is read before the error word is waited on (one memory round trip)
+    int2 w0, w1;
+    wave_range(d.face_wave, d.face_waves, d.gran4, wave, w0, w1);
+    // after a flagged mesh update the face lists may be incomplete: leave D[t] untouched
+    if (*d.err != 0)
+        return;
+    if (w0.x >= w1.x)
+        return;
+    FaceGather g{d, t, -1, 0.0f, 0.0f};
+    gather_wave(g, d.face_start, w0, w1, lane, lds);
 }
 
 // p(c) = far + 0.98 * sum W^bem (*) (N, D) over all 16 taps; records listener samples.
-__device__ __forceinline__ void near_wave(const SceneStep &d, int wave, int lane, float *__restrict__ vals)
+struct NearGather
+{
+    struct Index
+    {
+        int p, rec;
+    };
+    const SceneStep &d;
+    float *g;
+    size_t nn;
+    int t, lc;
+    unsigned cell;
+    float fv;
+    __device__ __forceinline__ Index load(int p) const { return Index{p, d.c3_pairs[p]}; }
+    __device__ __forceinline__ void conv(Index i, int n, int lane, float4 *term, float *vals) const
+    {
+        vals[lane] = conv_round<0, false>(d.owb ? d.owb : d.wb, d.owb ? d.osb : d.sb, d.owb ? i.p : i.rec, i.rec / GC, n,
+                                          d.wn, d.wd, lane, term, nullptr);
+    }
+    __device__ __forceinline__ void early(int s, bool in)
+    {
+        cell = in ? (unsigned)d.c3_cells[s] : ~0u;
+        fv = in ? d.far[s] : 0.0f;
+    }
+    __device__ __forceinline__ void late() {}
+    __device__ __forceinline__ void done(int s, float acc) const
+    {
+        const float v = (float)((double)fv + (double)acc * 0.98);
+        if (cell < nn)
+            g[cell] = v;
+        if (d.out)
+            for (int l = 0; l < d.a.n_listen; l++)
+                if (__builtin_amdgcn_readlane(lc, l) == s)
+                    d.out[(size_t)(t - d.a.t0) * d.out_stride + l] = v;
+    }
+};
+__device__ __forceinline__ void near_wave(const SceneStep &d, int wave, int lane, GatherLds<float> &lds)
 {
     // the wave map is read before the error word is waited on (in bounds either way), and lane l
     // reads listener l's C3 index: the table set with the listeners, or, for lists that move with
     // the mesh (lc3 null), this update's map of the listener's cell
+    const int nw = gran_waves(d.c3_waves, d.gran3);
     int2 w0 = {0, 0}, w1 = {0, 0};
-    if (wave < d.c3_waves)
-    {
-        w0 = reinterpret_cast<const int2 *>(d.c3_wave)[wave];
-        w1 = reinterpret_cast<const int2 *>(d.c3_wave)[wave + 1];
-    }
+    if (wave < nw)
+        wave_range(d.c3_wave, d.c3_waves, d.gran3, wave, w0, w1);
     int lc = -1;
     if (d.out && lane < d.a.n_listen)
         lc = d.lc3 ? d.lc3[lane] : d.c3_index[d.lcell[lane]];
@@ -322,50 +435,14 @@ __device__ __forceinline__ void near_wave(const SceneStep &d, int wave, int lane
     const int t = d.st->t;
     const size_t nn = (size_t)d.a.N * d.a.N * d.a.N;
     float *g = d.grid3 + (size_t)(((t % 3) + 3) % 3) * nn;
-    if (wave < d.c3_waves)
+    if (wave < nw)
     {
-        const int c0 = w0.x, q0 = w0.y, c1 = w1.x, q1 = w1.y;
-        if (c0 >= c1)
+        if (w0.x >= w1.x)
             return;
-        const int cs = c0 + lane;
-        const bool leader = cs < c1;
-        // every index of the wave's first round is loaded at once, then what they point to
-        const int m0 = leader ? d.c3_start[cs] : 0, m1 = leader ? d.c3_start[cs + 1] : 0;
-        const unsigned cell = leader ? (unsigned)d.c3_cells[cs] : ~0u;
-        const float fv = leader ? d.far[cs] : 0.0f;
-        int rec = q0 + lane < q1 ? d.c3_pairs[q0 + lane] : -1;
-        float acc = 0.0f;
-        for (int base = q0; base < q1; base += WAVE)
-        {
-            const int p = base + lane;
-            // the next round's index is loaded now, beside this round's records
-            const int rec_next = p + WAVE < q1 ? d.c3_pairs[p + WAVE] : -1;
-            float v = 0.0f;
-            if (p < q1)  // rec >= 0 exactly then; the list-ordered record does not wait for rec
-            {
-                const int tri = rec / GC;
-                const uint32_t *w = d.owb ? d.owb + (size_t)p * STEPS : d.wb + (size_t)rec * STEPS;
-                const float2 sc = d.owb ? d.osb[p] : d.sb[rec];
-                v = conv_pair<0, false>(w, sc, d.wn + tri * STEPS, d.wd + tri * STEPS);
-            }
-            vals[lane] = v;
-            wave_sync();
-            acc = round_sum(acc, vals, max(m0, base) - base, min(m1, base + WAVE) - base);
-            wave_sync();
-            rec = rec_next;
-        }
-        const float v = (float)((double)fv + (double)acc * 0.98);
-        if (leader && cell < nn)
-            g[cell] = v;
-        if (d.out)
-            for (int l = 0; l < d.a.n_listen; l++)
-            {
-                const int c3l = __shfl(lc, l);  // every lane takes part
-                if (leader && c3l == cs)
-                    d.out[(size_t)(t - d.a.t0) * d.out_stride + l] = v;
-            }
+        NearGather ng{d, g, nn, t, lc, ~0u, 0.0f};
+        gather_wave(ng, d.c3_start, w0, w1, lane, lds);
     }
-    else if (d.out && wave == d.c3_waves)
+    else if (d.out && wave == nw)
     {
         // listeners outside the corrected region read the grid directly (no wave writes them)
         if (lane < d.a.n_listen && lc < 0)
@@ -381,24 +458,23 @@ __global__ __launch_bounds__(256) void k_windows(SceneStep d, int back)
 
 __global__ __launch_bounds__(TB) void k_far(SceneStep d, int xper)
 {
-    __shared__ __align__(16) float vals[WPB][WAVE];
+    __shared__ GatherLds<float> lds[WPB];
     const int wid = threadIdx.x >> 6;
-    far_wave(d, xcd_wave(xper, wid), threadIdx.x & 63, vals[wid]);
+    far_wave(d, xcd_wave(xper, wid), threadIdx.x & 63, lds[wid]);
 }
 
 __global__ __launch_bounds__(TB) void k_dirichlet(SceneStep d)
 {
-    __shared__ __align__(16) float vals[WPB][WAVE];
-    __shared__ __align__(16) float facs[WPB][WAVE];
+    __shared__ GatherLds<float2> lds[WPB];
     const int wid = threadIdx.x >> 6;
-    dirichlet_wave(d, blockIdx.x * WPB + wid, threadIdx.x & 63, vals[wid], facs[wid]);
+    dirichlet_wave(d, blockIdx.x * WPB + wid, threadIdx.x & 63, lds[wid]);
 }
 
 __global__ __launch_bounds__(TB) void k_near(SceneStep d, int xper)
 {
-    __shared__ __align__(16) float vals[WPB][WAVE];
+    __shared__ GatherLds<float> lds[WPB];
     const int wid = threadIdx.x >> 6;
-    near_wave(d, xcd_wave(xper, wid), threadIdx.x & 63, vals[wid]);
+    near_wave(d, xcd_wave(xper, wid), threadIdx.x & 63, lds[wid]);
 }
 
 __global__ void k_listen_direct(SceneStep d)
@@ -492,33 +568,32 @@ __global__ __launch_bounds__(256) void k_batch_windows(const SceneStep *__restri
 
 __global__ __launch_bounds__(TB) void k_batch_far(const SceneStep *__restrict__ ds, BatchMap m)
 {
-    __shared__ __align__(16) float vals[WPB][WAVE];
+    __shared__ GatherLds<float> lds[WPB];
     int sc, lb;
     if (!batch_block(m, sc, lb))
         return;
     const int wid = threadIdx.x >> 6;
-    far_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, vals[wid]);
+    far_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, lds[wid]);
 }
 
 __global__ __launch_bounds__(TB) void k_batch_dirichlet(const SceneStep *__restrict__ ds, BatchMap m)
 {
-    __shared__ __align__(16) float vals[WPB][WAVE];
-    __shared__ __align__(16) float facs[WPB][WAVE];
+    __shared__ GatherLds<float2> lds[WPB];
     int sc, lb;
     if (!batch_block(m, sc, lb))
         return;
     const int wid = threadIdx.x >> 6;
-    dirichlet_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, vals[wid], facs[wid]);
+    dirichlet_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, lds[wid]);
 }
 
 __global__ __launch_bounds__(TB) void k_batch_near(const SceneStep *__restrict__ ds, BatchMap m)
 {
-    __shared__ __align__(16) float vals[WPB][WAVE];
+    __shared__ GatherLds<float> lds[WPB];
     int sc, lb;
     if (!batch_block(m, sc, lb))
         return;
     const int wid = threadIdx.x >> 6;
-    near_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, vals[wid]);
+    near_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, lds[wid]);
 }
 
 __global__ void k_batch_advance(const SceneStep *__restrict__ ds, int n)
@@ -533,8 +608,11 @@ inline int blocks_for_waves(long long waves) { return waves > 0 ? (int)((waves +
 // blocks per XCD of a gather launch over `waves` waves (the launch has 8 times as many)
 inline int xcd_per(long long waves) { return (blocks_for_waves(waves) + 7) / 8; }
 
-long long far_waves(const SceneStep &d) { return (long long)d.c3_waves + (d.neumann ? (d.a.nt + WAVE - 1) / WAVE : 0); }
-long long near_waves(const SceneStep &d) { return (long long)d.c3_waves + (d.out ? 1 : 0); }
+long long far_waves(const SceneStep &d)
+{
+    return (long long)gran_waves(d.c3_waves, d.gran3) + (d.neumann ? (d.a.nt + WAVE - 1) / WAVE : 0);
+}
+long long near_waves(const SceneStep &d) { return (long long)gran_waves(d.c3_waves, d.gran3) + (d.out ? 1 : 0); }
 }  // namespace
 
 int batch_blocks(const SceneStep &d, BatchKernel k)
@@ -549,7 +627,7 @@ int batch_blocks(const SceneStep &d, BatchKernel k)
     case BatchKernel::Far:
         return blocks_for_waves(far_waves(d));
     case BatchKernel::Dirichlet:
-        return blocks_for_waves(d.face_waves);
+        return blocks_for_waves(gran_waves(d.face_waves, d.gran4));
     case BatchKernel::Near:
         return blocks_for_waves(near_waves(d));
     }
@@ -575,7 +653,7 @@ hipError_t launch_dirichlet(const SceneStep &d, hipStream_t s)
     // plain block order: the heavy face lists of finely meshed objects sit together in the wave
     // range, and round-robin spreads them over the XCDs (the contiguous mapping of the C3 gathers
     // cut this kernel's HBM traffic from 47.6 to 39.7 MB but raised its time from 19.1 to 21.6 us)
-    k_dirichlet<<<blocks_for_waves(d.face_waves), TB, 0, s>>>(d);
+    k_dirichlet<<<blocks_for_waves(gran_waves(d.face_waves, d.gran4)), TB, 0, s>>>(d);
     return hipGetLastError();
 }
 

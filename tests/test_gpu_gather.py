@@ -1,0 +1,71 @@
+"""The segmented gathers of the step: lists shorter and longer than a round (64 pairs) and a chunk
+(256), against the oracle; and one, two or four wave-map entries per wave (chosen by the number of
+waves a launch has), against each other. All bit for bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+N, H, C = 20, 0.01, 343.0
+DT = float(np.float32(H / (np.sqrt(3.0) * C)))
+
+
+def _cluster(n, seed=0, spread=0.02):
+    """n separate small triangles around the grid's centre."""
+    rng = np.random.default_rng(seed)
+    c = N * H / 2 + rng.uniform(-spread, spread, (n, 1, 3))
+    v = (c + rng.uniform(-0.003, 0.003, (n, 3, 3))).reshape(-1, 3)
+    return v.astype(np.float32), np.arange(3 * n, dtype=np.int32).reshape(n, 3)
+
+
+# pairs per cell / per triangle: all lists of one pair; one list of 63, 64, 65, 255, 257 pairs per
+# triangle and cell (every triangle in the same cell); 600 triangles over several cells
+@pytest.mark.parametrize("n,spread", [(1, 0.02), (2, 0.02), (63, 1e-4), (64, 1e-4), (65, 1e-4), (255, 1e-4),
+                                      (257, 1e-4), (600, 0.02)])
+def test_list_lengths_against_the_oracle(amd, oracle_mod, n, spread):
+    import torch
+    v, f = _cluster(n, seed=n, spread=spread)
+    g = amd.PPPMSolver(N, H, DT, (0, 0, 0), 0, 0.83, C)
+    o = oracle_mod.Oracle(N, H, DT, (0, 0, 0), C, 0.83, oracle_mod.FP64)
+    g.set_mesh(v, f)
+    o.set_mesh(v, f)
+    rng = np.random.default_rng(7)
+    # separate triangles in one cell couple strongly: short runs of small inputs stay finite
+    steps = 20
+    acc = rng.standard_normal((steps, n)).astype(np.float32)
+    out = torch.zeros(steps, 2, device="cuda")
+    lis = [(N // 2, N // 2, N // 2), (N // 2 + 3, N // 2, N // 2 - 2)]
+    g.run(torch.from_numpy(acc).cuda(), steps, lis, out)
+    ref = np.zeros((steps, 2), np.float32)
+    for i in range(steps):
+        o.step(acc[i])
+        ref[i] = [o.read(*x) for x in lis]
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+    assert np.array_equal(g.get_grid(0).view(np.uint32).reshape(-1), o.grid(0).view(np.uint32).reshape(-1))
+    for a, b in zip(g.get_history(), o.history()):
+        assert np.array_equal(a.view(np.uint32), np.asarray(b).view(np.uint32).reshape(a.shape))
+
+
+@pytest.mark.parametrize("n_scenes", [1, 3, 8])
+def test_entries_per_wave_agree(amd, scenes_mod, n_scenes):
+    """Scenes of about 8000 face entries each: alone one entry per wave, together two or four."""
+    import torch
+    sc = [scenes_mod.c3_scene(56, 4, seed=i, steps=6) for i in range(n_scenes)]
+
+    def solvers():
+        s = [amd.PPPMSolver(x.res, x.dl, x.dt, x.min_pos, 0, 0.83, x.c) for x in sc]
+        for a, x in zip(s, sc):
+            a.set_mesh(x.verts, x.tris)
+        return s
+    rng = np.random.default_rng(1)
+    acc = [torch.from_numpy(rng.standard_normal((6, len(x.tris))).astype(np.float32)).cuda() for x in sc]
+    lis = [x.listener for x in sc]
+    together = solvers()
+    out = torch.zeros(6, n_scenes, device="cuda")
+    amd.PPPMBatch(together).run(acc, 6, lis, out)
+    for i, s in enumerate(solvers()):
+        one = torch.zeros(6, 1, device="cuda")
+        s.run(acc[i], 6, [lis[i]], one)
+        assert torch.equal(one[:, 0].view(torch.int32), out[:, i].contiguous().view(torch.int32))
+        assert np.array_equal(s.get_grid(0).view(np.uint32), together[i].get_grid(0).view(np.uint32))
+        for a, b in zip(s.get_history(), together[i].get_history()):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
