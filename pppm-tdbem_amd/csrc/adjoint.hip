@@ -25,6 +25,7 @@
 // base cell it is a corner of), so each output has one writer and the sums have a fixed order.
 // The reverse time index lives in device memory, so a captured graph replays any step.
 #include "internal.hpp"
+#include "scene_device.hpp"
 
 #include <algorithm>
 
@@ -563,18 +564,13 @@ __global__ __launch_bounds__(BLK) void k_adj(AdjScene d)
     adj_kernel<KIND>(d, (int)blockIdx.x);
 }
 
-// Batched: one launch covers the blocks of every scene; virtual block v belongs to scene
-// m.scene_of[v] as its local block v - m.first[scene]. Blocks go to the 8 XCDs in turn and block
-// b takes virtual block (b % 8) * m.per + b / 8, so each XCD works through one contiguous run of
-// scenes.
+// Batched: one launch covers the blocks of every scene (map_block)
 template <int KIND>
 __global__ __launch_bounds__(BLK) void k_batch_adj(const AdjScene *__restrict__ ds, BatchMap m)
 {
-    const int v = (int)(blockIdx.x & 7) * m.per + (int)(blockIdx.x >> 3);
-    if (v >= m.total)
-        return;
-    const int sc = m.scene_of[v];
-    adj_kernel<KIND>(ds[sc], v - m.first[sc]);
+    int sc, lb;
+    if (map_block(m, (int)blockIdx.x, sc, lb))
+        adj_kernel<KIND>(scene_desc(ds, sc), lb);
 }
 
 __global__ void k_batch_adj_back(const AdjScene *__restrict__ ds, int n)

@@ -52,7 +52,8 @@ struct pppm_batch
     std::vector<int> variant;  // FDTD interior variant per scene
     DBuf<SceneStep> descs;
     DBuf<FdtdScene> fdescs;
-    Map m_fdtd, m_tile[kFdtdVariants], m_win, m_far, m_dir, m_near;
+    Map m_fdtd, m_tile[kFdtdVariants], m_win, m_far, m_ffar, m_dir, m_near;
+    bool face_far = false;  // the face far field takes a launch of its own (face_far_pass)
     // batched adjoint: scene table and one block map per reverse-step kernel
     DBuf<AdjScene> adescs;
     Map m_adj[kAdjKernels];
@@ -205,21 +206,50 @@ int collect_spans(pppm_batch *b)
     return PPPM_OK;
 }
 
+// windows of the next step from the rings (a fused step leaves the next one's behind)
+int enqueue_batch_windows(pppm_batch *b)
+{
+    BCK(launch_batch(BatchKernel::Windows, b->descs.p, b->m_win.view(), b->stream));
+    return PPPM_OK;
+}
+
+int enqueue_batch_dirichlet(pppm_batch *b)
+{
+    if (b->face_far)
+        BCK(launch_batch(BatchKernel::FaceFar, b->descs.p, b->m_ffar.view(), b->stream));
+    BCK(launch_batch(b->face_far ? BatchKernel::DirichletOnly : BatchKernel::Dirichlet, b->descs.p, b->m_dir.view(),
+                     b->stream));
+    return PPPM_OK;
+}
+
 int enqueue_batch_step(pppm_batch *b)
 {
+    if (!b->timing)
+    {
+        // three launches, as a single scene's step: the FDTD beside the far-field sums (tiled
+        // interiors before it), the Dirichlet update, the near field with the next windows
+        for (int v = 1; v < kFdtdVariants; v++)
+            if (b->m_tile[v].total > 0)
+                BCK(launch_batch_tile(v, b->fdescs.p, b->m_tile[v].view(), b->stream));
+        BCK(launch_batch_head(b->descs.p, b->m_far.view(), b->fdescs.p, b->m_fdtd.view(), b->stream));
+        BRC(enqueue_batch_dirichlet(b));
+        BCK(launch_batch_near(b->descs.p, b->m_near.view(), b->m_win.view(), b->stream));
+        return PPPM_OK;
+    }
+    // a span per phase: a launch each
     int sp = span_begin(b, 0);
     BRC(enqueue_fdtd(b));
     span_end(b, sp);
     const int n = (int)b->sc.size();
     sp = span_begin(b, 1);
-    BCK(launch_batch(BatchKernel::Windows, b->descs.p, b->m_win.view(), b->stream));
+    BRC(enqueue_batch_windows(b));
     BCK(launch_batch_advance(b->descs.p, n, b->stream));
     span_end(b, sp);
     sp = span_begin(b, 2);
     BCK(launch_batch(BatchKernel::Far, b->descs.p, b->m_far.view(), b->stream));
     span_end(b, sp);
     sp = span_begin(b, 3);
-    BCK(launch_batch(BatchKernel::Dirichlet, b->descs.p, b->m_dir.view(), b->stream));
+    BRC(enqueue_batch_dirichlet(b));
     span_end(b, sp);
     sp = span_begin(b, 4);
     BCK(launch_batch(BatchKernel::Near, b->descs.p, b->m_near.view(), b->stream));
@@ -341,26 +371,35 @@ int pppm_batch_run(pppm_batch *b, const float *const *neumann_series, const long
         w3 += d.c3_waves;
         w4 += d.face_waves;
     }
-    for (SceneStep &d : hd)
+    b->face_far = face_far_pass(w4);
+    for (int i = 0; i < n; i++)
     {
+        const pppm_solver *s = b->sc[i];
+        SceneStep &d = hd[i];
         d.gran3 = gather_gran(w3);
         d.gran4 = gather_gran(w4);
+        d.fused = d.win2 = b->timing ? 0 : 1;
+        d.ffar = b->face_far ? s->ffar.p : nullptr;
     }
     BCK(b->descs.ensure(n));
     BCK(hipMemcpyAsync(b->descs.p, hd.data(), n * sizeof(SceneStep), hipMemcpyHostToDevice, b->stream));
-    std::vector<int> nw(n), nf(n), nd(n), nn(n);
+    std::vector<int> nw(n), nf(n), nff(n), nd(n), nn(n);
     for (int i = 0; i < n; i++)
     {
         nw[i] = batch_blocks(hd[i], BatchKernel::Windows);
         nf[i] = batch_blocks(hd[i], BatchKernel::Far);
+        nff[i] = batch_blocks(hd[i], BatchKernel::FaceFar);
         nd[i] = batch_blocks(hd[i], BatchKernel::Dirichlet);
         nn[i] = batch_blocks(hd[i], BatchKernel::Near);
     }
     BRC(build_map(b, b->m_win, nw));
     BRC(build_map(b, b->m_far, nf));
+    BRC(build_map(b, b->m_ffar, nff));
     BRC(build_map(b, b->m_dir, nd));
     BRC(build_map(b, b->m_near, nn));
     BRC(build_fdtd(b));
+    if (!b->timing)
+        BRC(enqueue_batch_windows(b));
 
     int done = 0;
     if (use_graph && !b->timing)

@@ -14,7 +14,8 @@
 // (grids beyond the Infinity Cache) the interior is instead marched along x by its own
 // launch before the shell launch (k_fdtd_march). t is read from device memory (so the
 // launches can be replayed from a graph); a one-thread kernel advances it after.
-#include "internal.hpp"
+#include "fdtd_device.hpp"
+#include "scene_device.hpp"
 
 #include <algorithm>
 
@@ -24,127 +25,8 @@ namespace pppm_amd
 namespace
 {
 
-constexpr int BLK = 256;
 // interior edge (N - 4) from which the interior is marched along x instead of one thread per cell
 constexpr int kMarchMin = 128;
-
-__device__ inline float *level(float *g3, int t, int rel, size_t nn)
-{
-    int l = ((t + rel) % 3 + 3) % 3;
-    return g3 + (size_t)l * nn;
-}
-
-// Solve4x4Linear (fdtd.cu:36-86): cofactor inverse in FP32, FP64 reciprocal of the determinant.
-__device__ inline void solve4(const float a[4][4], const float b[4], float res[4])
-{
-    float s0 = a[0][0] * a[1][1] - a[1][0] * a[0][1];
-    float s1 = a[0][0] * a[1][2] - a[1][0] * a[0][2];
-    float s2 = a[0][0] * a[1][3] - a[1][0] * a[0][3];
-    float s3 = a[0][1] * a[1][2] - a[1][1] * a[0][2];
-    float s4 = a[0][1] * a[1][3] - a[1][1] * a[0][3];
-    float s5 = a[0][2] * a[1][3] - a[1][2] * a[0][3];
-    float c5 = a[2][2] * a[3][3] - a[3][2] * a[2][3];
-    float c4 = a[2][1] * a[3][3] - a[3][1] * a[2][3];
-    float c3 = a[2][1] * a[3][2] - a[3][1] * a[2][2];
-    float c2 = a[2][0] * a[3][3] - a[3][0] * a[2][3];
-    float c1 = a[2][0] * a[3][2] - a[3][0] * a[2][2];
-    float c0 = a[2][0] * a[3][1] - a[3][0] * a[2][1];
-    float invdet = (float)(1.0 / (double)(s0 * c5 - s1 * c4 + s2 * c3 + s3 * c2 - s4 * c1 + s5 * c0));
-    float inv[4][4];
-    inv[0][0] = (a[1][1] * c5 - a[1][2] * c4 + a[1][3] * c3) * invdet;
-    inv[0][1] = (-a[0][1] * c5 + a[0][2] * c4 - a[0][3] * c3) * invdet;
-    inv[0][2] = (a[3][1] * s5 - a[3][2] * s4 + a[3][3] * s3) * invdet;
-    inv[0][3] = (-a[2][1] * s5 + a[2][2] * s4 - a[2][3] * s3) * invdet;
-    inv[1][0] = (-a[1][0] * c5 + a[1][2] * c2 - a[1][3] * c1) * invdet;
-    inv[1][1] = (a[0][0] * c5 - a[0][2] * c2 + a[0][3] * c1) * invdet;
-    inv[1][2] = (-a[3][0] * s5 + a[3][2] * s2 - a[3][3] * s1) * invdet;
-    inv[1][3] = (a[2][0] * s5 - a[2][2] * s2 + a[2][3] * s1) * invdet;
-    inv[2][0] = (a[1][0] * c4 - a[1][1] * c2 + a[1][3] * c0) * invdet;
-    inv[2][1] = (-a[0][0] * c4 + a[0][1] * c2 - a[0][3] * c0) * invdet;
-    inv[2][2] = (a[3][0] * s4 - a[3][1] * s2 + a[3][3] * s0) * invdet;
-    inv[2][3] = (-a[2][0] * s4 + a[2][1] * s2 - a[2][3] * s0) * invdet;
-    inv[3][0] = (-a[1][0] * c3 + a[1][1] * c1 - a[1][2] * c0) * invdet;
-    inv[3][1] = (a[0][0] * c3 - a[0][1] * c1 + a[0][2] * c0) * invdet;
-    inv[3][2] = (-a[3][0] * s3 + a[3][1] * s1 - a[3][2] * s0) * invdet;
-    inv[3][3] = (a[2][0] * s3 - a[2][1] * s1 + a[2][2] * s0) * invdet;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-    {
-        float r = 0;
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            r += inv[i][j] * b[j];
-        res[i] = r;
-    }
-}
-
-// ab_condition_solve (fdtd.cu:88-137) for one shell cell
-__device__ inline void abc_cell(float *g, const float *gm, float *gp, int N, int i, int j, int k, const FdtdParams &p)
-{
-    const int co[3] = {i, j, k};
-    int judge[3];
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-        judge[d] = -((int)(co[d] == 1)) + ((int)(co[d] == N - 2));
-    const int strd[3] = {N * N, N, 1};
-    const int me = lin3(i, j, k, N);
-    const float dt = p.dt, h = p.h, c = p.c;
-    float a[4][4], b[4];
-    float coef = c * c * dt * dt / (h * h);
-    a[3][3] = 1;
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-        a[3][d] = -coef * (float)(judge[d] != 0);
-    const float gc = g[me], gmc = gm[me];
-    b[3] = -gmc + 2 * gc - coef * (6 * gc);
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-        b[3] += coef * g[me + strd[d]] * (float)(judge[d] <= 0) + coef * g[me - strd[d]] * (float)(judge[d] >= 0);
-    float coef1 = 1 / (dt * dt), coef2 = c / (2 * h * dt), coef3 = -(c * c) / (2 * h * h);
-#pragma unroll
-    for (int idx = 0; idx < 3; idx++)
-    {
-        const int x = idx, y = (idx + 1) % 3, z = (idx + 2) % 3;
-        a[idx][3] = coef1;
-        a[idx][x] = coef2;
-        a[idx][y] = coef3 * (float)(judge[y] != 0);
-        a[idx][z] = coef3 * (float)(judge[z] != 0);
-        b[idx] = -coef1 * (gmc - 2 * gc) +
-                 -coef2 * (g[me + strd[x]] * (float)(-(int)(judge[x] < 0)) +
-                           g[me - strd[x]] * (float)(-(int)(judge[x] > 0)) + gm[me + strd[x]] * (float)(-judge[x]) +
-                           gm[me - strd[x]] * (float)judge[x]) +
-                 -coef3 * (g[me + strd[y]] * (float)(judge[y] <= 0) + g[me - strd[y]] * (float)(judge[y] >= 0) +
-                           g[me + strd[z]] * (float)(judge[z] <= 0) + g[me - strd[z]] * (float)(judge[z] >= 0) -
-                           4 * gc);
-    }
-    float r[4];
-    solve4(a, b, r);
-    gp[me] = r[3];
-#pragma unroll
-    for (int d = 0; d < 3; d++)
-        if (judge[d] != 0)
-            g[me + judge[d] * strd[d]] = r[d];
-}
-
-// Leapfrog update of one interior cell from its six neighbours, in the reference's FP64
-// operation order: sum x-, x+, y-, y+, z-, z+, then -6 * centre; / h^2; 2 p + coef lap - p_prev
-__device__ __forceinline__ float leapfrog(float xm, float xp, float ym, float yp, float zm, float zp, float gc,
-                                          float gmv, const FdtdParams &p)
-{
-    double sum = 0;
-    sum += xm;
-    sum += xp;
-    sum += ym;
-    sum += yp;
-    sum += zm;
-    sum += zp;
-    sum -= 6 * gc;
-    const double lap = sum / p.hh;
-    double v = 2 * gc;
-    v += p.coef * lap;
-    v += -gmv;
-    return (float)v;
-}
 
 // Interior of a large grid: a block owns MTY x MTZ (y, z) columns of one chunk of x planes and
 // marches them along x, so the x-neighbours come from registers and the y/z neighbours of the
@@ -231,146 +113,14 @@ __global__ __launch_bounds__(MBLK) void k_fdtd_march(float *__restrict__ grid3, 
     march_columns(level(grid3, t, 0, nn), level(grid3, t, -1, nn), level(grid3, t, 1, nn), N, x0, x1, y, z0, p);
 }
 
-// Interior cells per thread of the thread-per-column path: XC consecutive x planes
-constexpr int XC = 4;
-
-// Interior columns (blocks [0, nb_inner)) and the ABC shell (the remaining blocks); nb_inner = 0
-// when the interior is marched by another kernel. blk: the block's index within this scene's
-// launch (or its share of a batched launch). An interior block covers 256 consecutive (y, z)
-// cells of one chunk of XC x planes (a chunk takes ceil((N-4)^2 / 256) blocks; every index is
-// 32-bit); each thread loads the XC + 2 values of its column, the y / z neighbours and the
-// previous level of its XC cells before it writes any of them, so the loads of XC cells are in
-// flight together.
-__device__ __forceinline__ void fdtd_block(float *__restrict__ grid3, const FdtdParams &p, int t, int blk,
-                                           int nb_inner)
-{
-    const int N = p.N;
-    const size_t nn = (size_t)N * N * N;
-    float *g = level(grid3, t, 0, nn);
-    const float *gm = level(grid3, t, -1, nn);
-    float *gp = level(grid3, t, 1, nn);
-    if (blk < nb_inner)
-    {
-        const unsigned M = N - 4, MM = M * M;
-        const unsigned bpp = (MM + BLK - 1) / BLK;
-        const unsigned xb = (unsigned)blk / bpp;
-        const unsigned q = ((unsigned)blk - xb * bpp) * BLK + threadIdx.x;
-        if (q < MM)
-        {
-            const unsigned yq = q / M;
-            const int y = 2 + (int)yq, z = 2 + (int)(q - yq * M), x0 = 2 + (int)xb * XC;
-            const int NN2 = N * N;
-            const int c0 = lin3(x0, y, z, N);
-            float col[XC + 2], ym[XC], yp[XC], zm[XC], zp[XC], pm[XC];
-#pragma unroll
-            for (int i = 0; i < XC + 2; i++)
-                col[i] = g[c0 + (min(x0 - 1 + i, N - 2) - x0) * NN2];  // planes past N - 2 are not used
-#pragma unroll
-            for (int i = 0; i < XC; i++)
-            {
-                const int me = c0 + (min(x0 + i, N - 3) - x0) * NN2;
-                ym[i] = g[me - N];
-                yp[i] = g[me + N];
-                zm[i] = g[me - 1];
-                zp[i] = g[me + 1];
-                pm[i] = gm[me];
-            }
-#pragma unroll
-            for (int i = 0; i < XC; i++)
-                if (x0 + i <= N - 3)
-                    // laplacian + update in FP64, sum order x-, x+, y-, y+, z-, z+, -6*centre (fdtd.cu:7-33)
-                    gp[c0 + i * NN2] = leapfrog(col[i], col[i + 2], ym[i], yp[i], zm[i], zp[i], col[i + 1], pm[i], p);
-        }
-    }
-    else
-    {
-        const int S = N - 2;
-        // z faces in 16 x 16 tiles of (x, y), padded: a block's cells share their neighbour rows
-        const int zt = (S - 2 + 15) / 16;
-        const int fx = 2 * S * S, fy = 2 * (S - 2) * S, fz = 2 * zt * zt * 256;
-        // blocks [nb_inner, nb_inner + nb_fxy): the x and y faces (rows along z, coalesced);
-        // the rest: the z faces, one cell per row, so their blocks are handed to the XCDs in
-        // contiguous runs of x planes and a plane's rows meet its neighbours' in one L2
-        const int b = blk - nb_inner;
-        const int nb_fxy = (fx + fy + BLK - 1) / BLK;
-        int idx;
-        if (b < nb_fxy)
-        {
-            idx = b * BLK + (int)threadIdx.x;
-            if (idx >= fx + fy)
-                idx = -1;
-        }
-        else
-        {
-            const int bz = b - nb_fxy, per = (fz + 8 * BLK - 1) / (8 * BLK);
-            idx = fx + fy + ((bz & 7) * per + (bz >> 3)) * BLK + (int)threadIdx.x;
-        }
-        int i = -1, j = 0, k = 0;
-        if (idx >= fx + fy + fz)
-            idx = -1;
-        if (idx < 0)
-            ;
-        else if (idx < fx)
-        {
-            const int side = idx / (S * S);
-            const int r = idx - side * (S * S);
-            i = side ? N - 2 : 1;
-            j = 1 + r / S;
-            k = 1 + r % S;
-        }
-        else if ((idx -= fx) < fy)
-        {
-            const int side = idx / ((S - 2) * S);
-            const int r = idx - side * ((S - 2) * S);
-            j = side ? N - 2 : 1;
-            i = 2 + r / S;
-            k = 1 + r % S;
-        }
-        else if ((idx -= fy) < fz)
-        {
-            const int side = idx / (zt * zt * 256);
-            const int r = idx - side * (zt * zt * 256);
-            const int tile = r >> 8, w = r & 255;
-            k = side ? N - 2 : 1;
-            i = 2 + (tile / zt) * 16 + (w >> 4);
-            j = 2 + (tile % zt) * 16 + (w & 15);
-            if (i > N - 3 || j > N - 3)
-                i = -1;
-        }
-        if (i >= 0)
-            abc_cell(g, gm, gp, N, i, j, k, p);
-    }
-}
-
-// The FDTD of one scene (interior blocks, then the ABC shell) and, with a fuse, the history
-// windows of the step's gathers (the last blocks; they read only the rings, which no FDTD block
-// writes).
+// The FDTD of one scene alone: the interior blocks, then the ABC shell
 __global__ __launch_bounds__(BLK) void k_fdtd_abc(float *__restrict__ grid3, FdtdParams p, const StepState *__restrict__ st,
-                                                  int nb_inner, int nb_fdtd, const int *__restrict__ skip, StepFuse f)
+                                                  int nb_inner, const int *__restrict__ skip, StatusOut f)
 {
-    // the update's status block for the host, before the skip: an update that raised an error
-    // is reported too
-    if (f.status_host && blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < f.status_n)
-        f.status_host[threadIdx.x] = f.status[threadIdx.x];
+    copy_status(f);
     if (skip && *skip)
         return;
-    const int t = st->t;
-    const int blk = (int)blockIdx.x;
-    if (blk < nb_fdtd)
-        fdtd_block(grid3, p, t, blk, nb_inner);
-    else
-    {
-        // windows for the step that follows (t + 1): row k = ring value at t + 1 - k (row 0 is
-        // overwritten by the far-field and Dirichlet launches before use)
-        const int i = (blk - nb_fdtd) * BLK + (int)threadIdx.x;
-        if (i < f.nt * STEPS)
-        {
-            const int tri = i / STEPS, k = i % STEPS;
-            const int slot = (t + 1 - k) & (RING - 1);
-            f.wn[i] = f.hn[tri * RING + slot];
-            f.wd[i] = f.hd[tri * RING + slot];
-        }
-    }
+    fdtd_block(grid3, p, st->t, (int)blockIdx.x, nb_inner);
 }
 
 // Interior of a small grid as LDS-staged 2.5D tiles: a block of TY x TZ threads owns TY x TZ
@@ -438,23 +188,21 @@ template <int TY, int TZ>
 __global__ __launch_bounds__(TY *TZ) void k_batch_tile(const FdtdScene *__restrict__ ds, BatchMap m)
 {
     __shared__ float lds[2 * (TY + 2) * (TZ + 2)];
-    const int v = (int)(blockIdx.x & 7) * m.per + (int)(blockIdx.x >> 3);
-    if (v >= m.total)
+    int sc, lb;
+    if (!map_block(m, (int)blockIdx.x, sc, lb))
         return;
-    const int sc = m.scene_of[v];
-    const FdtdScene &d = ds[sc];
-    tile_march<TY, TZ>(d.grid3, d.p, d.st->t, v - m.first[sc], d.xch, lds);
+    const FdtdScene d = scene_desc(ds, sc);
+    tile_march<TY, TZ>(d.grid3, d.p, d.st->t, lb, d.xch, lds);
 }
 
 // the ABC shell of every scene, plus the interior of the scenes stepped one thread per cell
 __global__ __launch_bounds__(BLK) void k_batch_fdtd(const FdtdScene *__restrict__ ds, BatchMap m)
 {
-    const int v = (int)(blockIdx.x & 7) * m.per + (int)(blockIdx.x >> 3);
-    if (v >= m.total)
+    int sc, lb;
+    if (!map_block(m, (int)blockIdx.x, sc, lb))
         return;
-    const int sc = m.scene_of[v];
-    const FdtdScene &d = ds[sc];
-    fdtd_block(d.grid3, d.p, d.st->t, v - m.first[sc], d.nb_inner);
+    const FdtdScene d = scene_desc(ds, sc);
+    fdtd_block(d.grid3, d.p, d.st->t, lb, d.nb_inner);
 }
 
 // get_damp (fdtd.cu:162-169)
@@ -593,8 +341,30 @@ hipError_t launch_batch_tile(int variant, const FdtdScene *ds, const BatchMap &m
     return hipGetLastError();
 }
 
+hipError_t launch_fdtd_march(float *grid3, const FdtdParams &p, const StepState *st, const int *skip, hipStream_t s,
+                             int &nb_inner)
+{
+    const int N = p.N;
+    const long long M = N - 4;
+    nb_inner = fdtd_inner_blocks(N);
+    if (M < kMarchMin)
+        return hipSuccess;
+    // about 2048 tiles or more; chunks of at least 16 planes (each chunk re-reads 2 planes)
+    MarchShape ms{};
+    ms.ntz = (N - 3) / MTZ + 1;  // z tiles [MTZ tz, MTZ tz + MTZ) up to z = N - 3
+    ms.nty = (int)((M + MTY - 1) / MTY);
+    const long long cols = (long long)ms.ntz * ms.nty;
+    const long long nxc = std::max<long long>(1, (2048 + cols - 1) / cols);
+    ms.xch = (int)std::max<long long>(16, (M + nxc - 1) / nxc);
+    ms.n_tiles = (int)(cols * ((M + ms.xch - 1) / ms.xch));
+    ms.n_blocks = (ms.n_tiles + 7) / 8 * 8;
+    k_fdtd_march<<<ms.n_blocks, MBLK, 0, s>>>(grid3, p, st, ms, skip);
+    nb_inner = 0;
+    return hipGetLastError();
+}
+
 hipError_t launch_fdtd(float *grid3, float *pml3, const FdtdParams &p, const StepState *st, hipStream_t s,
-                       const int *skip, const StepFuse *fuse)
+                       const int *skip, const StatusOut *status)
 {
     const int N = p.N;
     if (p.pml > 0)
@@ -604,33 +374,12 @@ hipError_t launch_fdtd(float *grid3, float *pml3, const FdtdParams &p, const Ste
         k_fdtd_pml<<<nb, BLK, 0, s>>>(grid3, pml3, p, st, skip);
         return hipGetLastError();
     }
-    const long long M = N - 4, S = N - 2;
-    int nb_inner = fdtd_inner_blocks(N);
-    if (M >= kMarchMin)
-    {
-        // about 2048 tiles or more; chunks of at least 16 planes (each chunk re-reads 2 planes)
-        MarchShape ms{};
-        ms.ntz = (N - 3) / MTZ + 1;  // z tiles [MTZ tz, MTZ tz + MTZ) up to z = N - 3
-        ms.nty = (int)((M + MTY - 1) / MTY);
-        const long long cols = (long long)ms.ntz * ms.nty;
-        const long long nxc = std::max<long long>(1, (2048 + cols - 1) / cols);
-        ms.xch = (int)std::max<long long>(16, (M + nxc - 1) / nxc);
-        ms.n_tiles = (int)(cols * ((M + ms.xch - 1) / ms.xch));
-        ms.n_blocks = (ms.n_tiles + 7) / 8 * 8;
-        k_fdtd_march<<<ms.n_blocks, MBLK, 0, s>>>(grid3, p, st, ms, skip);
-        nb_inner = 0;
-    }
-    const long long zt = (S - 2 + 15) / 16;
-    const long long fxy = 2 * S * S + 2 * (S - 2) * S, fz = 2 * zt * zt * 256;
-    const int nb_shell = (int)((fxy + BLK - 1) / BLK) + 8 * (int)((fz + 8LL * BLK - 1) / (8LL * BLK));
-    StepFuse f{};
-    int nb_win = 0;
-    if (fuse && fuse->wn)
-    {
-        f = *fuse;
-        nb_win = (int)(((long long)f.nt * STEPS + BLK - 1) / BLK);
-    }
-    k_fdtd_abc<<<nb_inner + nb_shell + nb_win, BLK, 0, s>>>(grid3, p, st, nb_inner, nb_inner + nb_shell, skip, f);
+    int nb_inner = 0;
+    const hipError_t e = launch_fdtd_march(grid3, p, st, skip, s, nb_inner);
+    if (e != hipSuccess)
+        return e;
+    k_fdtd_abc<<<nb_inner + fdtd_shell_blocks(N), BLK, 0, s>>>(grid3, p, st, nb_inner, skip,
+                                                              status ? *status : StatusOut{});
     return hipGetLastError();
 }
 

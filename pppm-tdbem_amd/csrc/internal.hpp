@@ -12,10 +12,12 @@ namespace pppm_amd
 
 // Device-resident step state: t follows the reference's fdtd.t (-1 before the first step,
 // advanced right after the FDTD kernel, src/algorithm/fdtd.h:73-87).
+// A whole step runs as three launches that hand t on without one of its own: the first reads t
+// and steps to t + 1, the second writes next = t + 1, the third reads next and writes t.
 struct StepState
 {
     int t;
-    int pad;
+    int next;
 };
 
 // device-side error bits (reported through the status block)
@@ -37,24 +39,21 @@ struct FdtdParams
 };
 
 // ---------------------------------------------------------------- fdtd.hip
-// What the ABC-shell launch of a time step can do besides the FDTD: the gathers' history
-// windows for the step, in extra blocks (wn / wd as in step.hip's windows_item with back = 0).
-// wn == nullptr: nothing. (Advancing t in the same launch, by the last block to finish, cost more
-// than the one-thread kernel it saves: every block counted itself done on one atomic.)
-struct StepFuse
+// A mesh update's status block on its way to the host: the launch that steps the FDTD copies the n
+// ints of status to host (pinned memory; null: nothing)
+struct StatusOut
 {
-    const float *hn, *hd;
-    float *wn, *wd;
-    int nt;
-    // status_host != null: the launch also copies the status_n ints of status (the mesh
-    // update's status block) to status_host (pinned host memory), whether or not it steps
     const int *status;
-    int *status_host;
-    int status_n;
+    int *host;
+    int n;
 };
 // skip (may be null): as for launch_advance
 hipError_t launch_fdtd(float *grid3, float *pml3, const FdtdParams &p, const StepState *st, hipStream_t s,
-                       const int *skip = nullptr, const StepFuse *fuse = nullptr);
+                       const int *skip = nullptr, const StatusOut *status = nullptr);
+// marches the interior of a large grid (nb_inner = 0), or leaves it to nb_inner blocks of the
+// launch that follows
+hipError_t launch_fdtd_march(float *grid3, const FdtdParams &p, const StepState *st, const int *skip, hipStream_t s,
+                             int &nb_inner);
 // One scene of a batched FDTD step. nb_inner: blocks of its one-thread-per-cell interior in the
 // batched shell launch (0: the interior is marched by a tile launch); xch: x planes per tile.
 struct FdtdScene
@@ -332,6 +331,13 @@ struct SceneStep
     int face_waves;
     // wave-map entries (64 pairs each) a wave of the C3 gathers / the face gather takes
     int gran3, gran4;
+    // 0: a phase of its own; the time index is t and far holds the far field. 1: part of a step in
+    // three launches (launch_step_head, launch_dirichlet, launch_near); far holds the sums the far
+    // field subtracts from the pressure, which its readers subtract themselves.
+    int fused;
+    // the windows of step t are at (t & 1) * 16 * nt of wn / wd and the near-field launch writes
+    // those of step t + 1 to the other half; 0: one set, rewritten before every step
+    int win2;
     const int *face_start, *face_wave, *face_nbr, *face_slot;
     const uint32_t *wf, *wb, *fw;  // 16 x half2 {S_k, D_k} per record
     const float2 *sf, *sb, *fsc;   // scales
@@ -345,6 +351,8 @@ struct SceneStep
     const int *err;
     // histories and per-step buffers
     float *hn, *hd, *wn, *wd, *far;
+    // the triangles' face far field, formed by a launch of its own; null: by the Dirichlet update
+    float *ffar;
     const float *neumann;  // Neumann series (row t - t0), null: the ring slot is written elsewhere
     // listener recording: out[(t - t0) * out_stride + l] for l < a.n_listen (null: none); lc3
     // null: the listeners' C3 indices are read from c3_index (cell -> C3 index) per step
@@ -361,11 +369,19 @@ struct SceneStep
 // 141^3 / 20480 triangles (22k face entries) 2.71 / 2.51 / 2.58 ms for 32 steps; 64 scenes (111k
 // face, 42k C3 entries) 18.2 / 16.4 / 16.0 ms for 32 steps.
 constexpr int gather_gran(long long waves) { return waves >= 4 * 8192 ? 4 : waves >= 2 * 8192 ? 2 : 1; }
+// Whether the face far field takes a launch of its own before the Dirichlet update. Formed inside
+// it, its eight dependent loads per triangle cost the gather registers and time where the device is
+// full (64 scenes: 193 -> 169 + 11 us, 80k triangles in 64^3 grids: 399 -> 347 + 8 us); where it is
+// not, a launch more costs a step of 64^3 / 5120 triangles 4 of 25 us.
+constexpr bool face_far_pass(long long face_waves) { return face_waves >= 4 * 8192; }
 // history windows of the gathers: wn/wd[tri*16 + k] = ring value of time t - k, the value of tap k
 // (t: the step the gathers serve, the device time index plus 1 - back when the kernel runs: back =
 // 0 before the advance of a step, 1 after)
 hipError_t launch_windows(const SceneStep &d, int back, hipStream_t s);
 hipError_t launch_far(const SceneStep &d, hipStream_t s);
+// the first launch of a fused step: the FDTD (its interior too unless marched) and, beside it, the
+// far-field sums, which read only the histories, and the Neumann input
+hipError_t launch_step_head(const SceneStep &d, const FdtdParams &p, const StatusOut &status, hipStream_t s);
 hipError_t launch_dirichlet(const SceneStep &d, hipStream_t s);
 hipError_t launch_near(const SceneStep &d, hipStream_t s);
 hipError_t launch_listen_direct(const SceneStep &d, hipStream_t s);
@@ -399,9 +415,17 @@ enum class BatchKernel
 {
     Windows,
     Far,
-    Dirichlet,
+    FaceFar,
+    DirichletOnly,  // the face far field is there (FaceFar)
+    Dirichlet,      // forms it too
     Near
 };
+struct FdtdScene;
+// the batched form of launch_step_head: far blocks by the map mf, FDTD blocks by the map mb
+hipError_t launch_batch_head(const SceneStep *descs, const BatchMap &mf, const FdtdScene *fd, const BatchMap &mb,
+                             hipStream_t s);
+// the near field of every scene and, by the map mw, the windows of the next step
+hipError_t launch_batch_near(const SceneStep *descs, const BatchMap &mn, const BatchMap &mw, hipStream_t s);
 // blocks of one scene in a batched launch of kernel k
 int batch_blocks(const SceneStep &d, BatchKernel k);
 hipError_t launch_batch(BatchKernel k, const SceneStep *descs, const BatchMap &m, hipStream_t s);

@@ -580,11 +580,11 @@ int upload(pppm_solver *s, void *dst, const void *src, size_t bytes, int on_devi
 // per-device scratch array
 struct StepBufs
 {
-    float *wn, *wd, *far;
+    float *wn, *wd, *far, *ffar;
     const int *lcell, *lc3;
 };
 
-StepBufs own_bufs(pppm_solver *s) { return StepBufs{s->wn.p, s->wd.p, s->far.p, s->lcell.p, s->lc3.p}; }
+StepBufs own_bufs(pppm_solver *s) { return StepBufs{s->wn.p, s->wd.p, s->far.p, s->ffar.p, s->lcell.p, s->lc3.p}; }
 
 // the step kernels' view of the handle (neumann: series rows t - t0 or null; out: listener
 // samples, n_listen per step, or null)
@@ -631,6 +631,7 @@ SceneStep scene_step(const pppm_solver *s, const StepBufs &b, const float *neuma
     d.wn = b.wn;
     d.wd = b.wd;
     d.far = b.far;
+    d.ffar = b.ffar && face_far_pass(s->face_waves) ? b.ffar : nullptr;
     d.neumann = neumann;
     d.lcell = b.lcell;
     d.lc3 = b.lc3;
@@ -640,48 +641,58 @@ SceneStep scene_step(const pppm_solver *s, const StepBufs &b, const float *neuma
     return d;
 }
 
+// Where a step's history windows come from. A step of a series (First, then Next) leaves those of
+// the step after it behind, in the half it does not read itself: only the first builds its own.
+enum class Windows
+{
+    First,
+    Next,
+    Alone,  // builds its own and leaves none (one set of windows)
+};
+
 // one update_grid_and_face on the handle's stream; neumann is device memory (row t - t0).
 // timed: phase spans when timing is on (events are created on first use, so the
 // allocation-free path passes false)
 // status_event != null: the FDTD launch also copies the mesh update's status block to st_h and
 // the event is recorded right behind it (the caller has checked fused_status)
 int enqueue_step(pppm_solver *s, const StepBufs &b, const float *neumann, int t0, long long stride, int n_listen,
-                 float *out, bool timed = true, hipEvent_t status_event = nullptr)
+                 float *out, Windows win, bool timed = true, hipEvent_t status_event = nullptr)
 {
     const FdtdParams fp = fdtd_params(s);
-    const SceneStep d = scene_step(s, b, neumann, t0, stride, n_listen, out);
+    SceneStep d = scene_step(s, b, neumann, t0, stride, n_listen, out);
     // a step enqueued behind a mesh update does nothing if that update raises an error bit
     const int *skip = s->mesh_set ? d.err : nullptr;
-    int sp = timed ? span_begin(s, 0) : -1;
-    if (s->mesh_set && !s->use_pml)
-    {
-        // the ABC-shell launch also builds the gathers' history windows
-        StepFuse fuse{s->hn.p, s->hd.p, d.wn, d.wd, s->nt, nullptr, nullptr, 0};
-        if (status_event)
-        {
-            fuse.status = s->status.p;
-            fuse.status_host = s->st_hdev;
-            fuse.status_n = ST_N;
-        }
-        CK(launch_fdtd(s->grid.p, s->pmlbuf.p, fp, s->state.p, s->stream, skip, &fuse));
-        if (status_event)
-            CK(hipEventRecord(status_event, s->stream));
-        span_end(s, sp);
-    }
-    else
-    {
-        CK(launch_fdtd(s->grid.p, s->pmlbuf.p, fp, s->state.p, s->stream, skip));
-        span_end(s, sp);
-        if (s->mesh_set)
-            CK(launch_windows(d, 0, s->stream));
-    }
-    CK(launch_advance(s->state.p, s->stream, skip));
+    const StatusOut status = status_event ? StatusOut{s->status.p, s->st_hdev, ST_N} : StatusOut{};
     if (!s->mesh_set)
     {
+        CK(launch_fdtd(s->grid.p, s->pmlbuf.p, fp, s->state.p, s->stream, skip));
+        CK(launch_advance(s->state.p, s->stream, skip));
         if (out)
             CK(launch_listen_direct(d, s->stream));
         return PPPM_OK;
     }
+    timed = timed && s->timing;
+    if (!s->use_pml && !timed)
+    {
+        d.fused = 1;
+        d.win2 = win != Windows::Alone;
+        if (win != Windows::Next)
+            CK(launch_windows(d, 0, s->stream));
+        CK(launch_step_head(d, fp, status, s->stream));
+        if (status_event)
+            CK(hipEventRecord(status_event, s->stream));
+        CK(launch_dirichlet(d, s->stream));
+        CK(launch_near(d, s->stream));
+        return PPPM_OK;
+    }
+    // the PML, or a span per phase: a launch each
+    int sp = timed ? span_begin(s, 0) : -1;
+    CK(launch_fdtd(s->grid.p, s->pmlbuf.p, fp, s->state.p, s->stream, skip, &status));
+    if (status_event)
+        CK(hipEventRecord(status_event, s->stream));
+    span_end(s, sp);
+    CK(launch_windows(d, 0, s->stream));
+    CK(launch_advance(s->state.p, s->stream, skip));
     sp = timed ? span_begin(s, 1) : -1;
     CK(launch_far(d, s->stream));
     span_end(s, sp);
@@ -708,7 +719,7 @@ int check_handle(pppm_solver *s) { return s ? PPPM_OK : PPPM_ERR_ARG; }
 // neumann: device rows (row t - t0, stride; null: the ring slot is written elsewhere); out:
 // listener samples by a direct read (may be null). The caller advances t_host when it returns OK.
 int update_and_step(pppm_solver *s, const float *vsrc, const float *neumann, int t0, long long stride, int n_listen,
-                    float *out)
+                    float *out, Windows win)
 {
     auto &c = s->stc;
     if (!c.ev_status)
@@ -729,7 +740,7 @@ int update_and_step(pppm_solver *s, const float *vsrc, const float *neumann, int
         // the lists moved with this update: the near field looks the listeners' C3 indices up
         StepBufs b = own_bufs(s);
         b.lc3 = nullptr;
-        return enqueue_step(s, b, neumann, t0, stride, n_listen, out, true, fused_status ? c.ev_status : nullptr);
+        return enqueue_step(s, b, neumann, t0, stride, n_listen, out, win, true, fused_status ? c.ev_status : nullptr);
     };
     RC(step());
     CK(hipEventSynchronize(c.ev_status));
@@ -864,9 +875,10 @@ struct StaticChunk
 };
 int enqueue_static_chunk(void *p)
 {
+    // the windows of the first step are built before the graph is launched
     const StaticChunk &c = *static_cast<const StaticChunk *>(p);
     for (int i = 0; i < c.chunk; i++)
-        RC(enqueue_step(c.s, own_bufs(c.s), c.neumann, c.t0, c.stride, c.n_listen, c.out));
+        RC(enqueue_step(c.s, own_bufs(c.s), c.neumann, c.t0, c.stride, c.n_listen, c.out, Windows::Next));
     return PPPM_OK;
 }
 
@@ -904,9 +916,10 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
     if (verts_series && !kAsyncMovingStep)
         use_graph = 0;
     auto one_step = [&](int i) -> int {
+        const Windows win = i == 0 ? Windows::First : Windows::Next;
         if (verts_series && !kAsyncMovingStep)
             // the synchronous update with its status read overlapped with the step
-            return update_and_step(s, verts_series + (size_t)i * vstride, neumann_series, t0, stride, n_listen, out);
+            return update_and_step(s, verts_series + (size_t)i * vstride, neumann_series, t0, stride, n_listen, out, win);
         if (verts_series)
         {
             const int sp = span_begin(s, 4);
@@ -914,9 +927,9 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
             span_end(s, sp);
         }
         if (!verts_series)
-            return enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, out);
+            return enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, out, win);
         // with moving lists the listener is read by its own launch after the near field
-        RC(enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, nullptr));
+        RC(enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, nullptr, win));
         if (out)
             CK(launch_listen_direct(scene_step(s, own_bufs(s), nullptr, t0, stride, n_listen, out), s->stream));
         return PPPM_OK;
@@ -940,6 +953,14 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
         StaticChunk sc{s, neumann_series, t0, stride, n_listen, out, chunk};
         hipGraphExec_t ge = nullptr;
         int rc = solver_cached_graph(s, s->step_graphs, &key, sizeof key, enqueue_static_chunk, &sc, &ge);
+        if (rc == PPPM_OK && s->mesh_set && !s->use_pml)
+        {
+            SceneStep d = scene_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, out);
+            d.win2 = 1;
+            const hipError_t we = launch_windows(d, 0, s->stream);
+            if (we != hipSuccess)
+                rc = fail(s, PPPM_ERR_HIP, std::string("windows launch: ") + hipGetErrorString(we));
+        }
         for (; rc == PPPM_OK && done + chunk <= steps; done += chunk)
         {
             const hipError_t le = hipGraphLaunch(ge, s->stream);
@@ -1107,7 +1128,7 @@ int solver_cached_graph(pppm_solver *s, GraphCache &c, const void *key, size_t n
 SceneStep solver_scene_step(const pppm_solver *s, const float *neumann, int t0, long long stride, int n_listen,
                             float *out)
 {
-    return scene_step(s, StepBufs{s->wn.p, s->wd.p, s->far.p, s->lcell.p, s->lc3.p}, neumann, t0, stride, n_listen,
+    return scene_step(s, StepBufs{s->wn.p, s->wd.p, s->far.p, s->ffar.p, s->lcell.p, s->lc3.p}, neumann, t0, stride, n_listen,
                       out);
 }
 }  // namespace pppm_amd
@@ -1239,8 +1260,9 @@ int pppm_set_mesh(pppm_solver *s, const float *verts, int nv, const int *tris, i
     // dirichlet / neumann histories reset (pppm.h:88-91)
     CK(s->hn.ensure((size_t)nt * RING));
     CK(s->hd.ensure((size_t)nt * RING));
-    CK(s->wn.ensure((size_t)nt * STEPS));
-    CK(s->wd.ensure((size_t)nt * STEPS));
+    CK(s->wn.ensure(2 * (size_t)nt * STEPS));
+    CK(s->wd.ensure(2 * (size_t)nt * STEPS));
+    CK(s->ffar.ensure(nt));
     CK(s->nstage.ensure(nt));
     CK(hipMemsetAsync(s->hn.p, 0, (size_t)nt * RING * sizeof(float), s->stream));
     CK(hipMemsetAsync(s->hd.p, 0, (size_t)nt * RING * sizeof(float), s->stream));
@@ -1312,7 +1334,7 @@ int pppm_step(pppm_solver *s, const float *neumann, int on_device)
         nd = s->nstage.p;
     }
     const int t_new = s->t_host + 1;
-    RC(enqueue_step(s, own_bufs(s), nd, t_new, 0, 0, nullptr));
+    RC(enqueue_step(s, own_bufs(s), nd, t_new, 0, 0, nullptr, Windows::Alone));
     s->t_host = t_new;
     return PPPM_OK;
 }
@@ -1362,7 +1384,7 @@ int pppm_run_noalloc(pppm_solver *s, const float *neumann_series, long long stri
     CK(scratch_ptr(&base));
     unsigned char *sb = (unsigned char *)base;
     int *lcell = (int *)sb, *lc3 = (int *)sb + 64;
-    const StepBufs b{(float *)(sb + off_wn), (float *)(sb + off_wd), (float *)(sb + off_far), lcell, lc3};
+    const StepBufs b{(float *)(sb + off_wn), (float *)(sb + off_wd), (float *)(sb + off_far), nullptr, lcell, lc3};
     // every scratch entry a kernel reads is written earlier in the same call: the listener
     // table here, the windows by each step's window copy, the far field of the live C3 cells by
     // each step's far-field gather (the Dirichlet update and the near field read only those)
@@ -1371,7 +1393,7 @@ int pppm_run_noalloc(pppm_solver *s, const float *neumann_series, long long stri
     const int t0 = s->t_host + 1;
     float *out = n_listen > 0 ? out_dev : nullptr;
     for (int i = 0; i < steps; i++)
-        RC(enqueue_step(s, b, neumann_series, t0, stride, n_listen, out, false));
+        RC(enqueue_step(s, b, neumann_series, t0, stride, n_listen, out, Windows::Alone, false));
     s->t_host += steps;
     return PPPM_OK;
 }
@@ -1405,7 +1427,7 @@ int pppm_update_mesh_and_step(pppm_solver *s, const float *verts, const float *n
             nd = s->nstage.p;
         }
     }
-    RC(update_and_step(s, on_device ? verts : nullptr, nd, s->t_host + 1, 0, 0, nullptr));
+    RC(update_and_step(s, on_device ? verts : nullptr, nd, s->t_host + 1, 0, 0, nullptr, Windows::Alone));
     s->t_host++;
     return PPPM_OK;
 }
@@ -1484,7 +1506,7 @@ int pppm_reset(pppm_solver *s)
         CK(hipMemsetAsync(s->hn.p, 0, (size_t)s->nt * RING * sizeof(float), s->stream));
         CK(hipMemsetAsync(s->hd.p, 0, (size_t)s->nt * RING * sizeof(float), s->stream));
     }
-    static_assert(sizeof(StepState) == 2 * sizeof(int), "StepState is {t, pad}");
+    static_assert(sizeof(StepState) == 2 * sizeof(int), "StepState is {t, next}");
     CK(launch_put_ints(reinterpret_cast<int *>(s->state.p), 2, -1, 0, 0, 0, s->stream));
     s->t_host = -1;
     return PPPM_OK;

@@ -174,8 +174,8 @@ struct pppm_solver
     DBuf<uint32_t> owf, owb, ofw;
     DBuf<float2> osf, osb, ofsc;
 
-    DBuf<float> hn, hd, far, nstage;
-    DBuf<float> wn, wd;  // per-step history windows, 16 floats per triangle and field
+    DBuf<float> hn, hd, far, ffar, nstage;
+    DBuf<float> wn, wd;  // per-step history windows, 16 floats per triangle and field, two sets
     DBuf<int> lcell, lc3;
 
     // cell classification and fresh cells (GhostCellSolver cell_data / cell_data_old,

@@ -31,7 +31,11 @@
 //
 // Time index: all kernels read t from device memory (StepState), so one captured HIP
 // graph replays any step.
+#include "fdtd_device.hpp"
 #include "internal.hpp"
+#include "scene_device.hpp"
+
+#include <algorithm>
 
 namespace pppm_amd
 {
@@ -49,6 +53,8 @@ __device__ inline int xcd_wave(int per, int wid)
 {
     return ((int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3)) * WPB + wid;
 }
+
+__device__ inline int wave_in_block() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
 __device__ inline void wave_sync()
 {
@@ -167,8 +173,8 @@ __device__ __forceinline__ void gather_wave(G &g, const int *__restrict__ start,
 // map entries [gran * wave, gran * (wave + 1)) of a gather's wave map: its first segment and pair
 __device__ __forceinline__ void wave_range(const int *__restrict__ map, int waves, int gran, int wave, int2 &w0, int2 &w1)
 {
-    w0 = reinterpret_cast<const int2 *>(map)[gran * wave];
-    w1 = reinterpret_cast<const int2 *>(map)[min(gran * (wave + 1), waves)];
+    w0 = const_load(reinterpret_cast<const int2 *>(map) + gran * wave);
+    w1 = const_load(reinterpret_cast<const int2 *>(map) + min(gran * (wave + 1), waves));
 }
 __host__ __device__ inline int gran_waves(int waves, int gran) { return (waves + gran - 1) / gran; }
 
@@ -250,15 +256,20 @@ __device__ __forceinline__ float conv_round(const uint32_t *__restrict__ w16, co
 // not exist yet; the far-field launch writes the Neumann value and the Dirichlet update the
 // Dirichlet value into row 0 as into the ring), 1 after it (the phase entry points: the ring
 // holds them).
-__device__ __forceinline__ void windows_item(const SceneStep &d, int back, int i)
+// windows of step t in their half of wn / wd
+__device__ __forceinline__ size_t window_base(const SceneStep &d, int t)
+{
+    return d.win2 && (t & 1) ? (size_t)d.a.nt * STEPS : 0;
+}
+__device__ __forceinline__ void windows_item(const SceneStep &d, int tn, int i)
 {
     if (i >= d.a.nt * STEPS || (d.err && *d.err))
         return;
     const int tri = i / STEPS, k = i % STEPS;
-    const int tn = d.st->t - back + 1;  // t of the step the gathers serve
     const int slot = (tn - k) & (RING - 1);
-    d.wn[i] = d.hn[tri * RING + slot];
-    d.wd[i] = d.hd[tri * RING + slot];
+    const size_t o = window_base(d, tn) + i;
+    d.wn[o] = d.hn[tri * RING + slot];
+    d.wd[o] = d.hd[tri * RING + slot];
 }
 
 // far(c) = p(c) - sum_pairs W^fdtd (*) (N, D). W^fdtd has tap 0 == 0 (pppm_cache.cu:111),
@@ -271,6 +282,7 @@ struct FarGather
         int p, rec;
     };
     const SceneStep &d;
+    const float *wn, *wd;
     const float *g;
     size_t nn;
     unsigned cell;
@@ -278,12 +290,15 @@ struct FarGather
     __device__ __forceinline__ Index load(int p) const { return Index{p, d.c3_pairs[p]}; }
     __device__ __forceinline__ void conv(Index i, int n, int lane, float4 *term, float *vals) const
     {
-        vals[lane] = conv_round<1, false>(d.owf ? d.owf : d.wf, d.owf ? d.osf : d.sf, d.owf ? i.p : i.rec, i.rec / GC, n,
-                                          d.wn, d.wd, lane, term, nullptr);
+        vals[lane] = conv_round<1, false>(d.owf ? d.owf : d.wf, d.owf ? d.osf : d.sf, d.owf ? i.p : i.rec, i.rec / GC, n, wn,
+                                          wd, lane, term, nullptr);
     }
-    __device__ __forceinline__ void early(int s, bool in) { cell = in ? (unsigned)d.c3_cells[s] : ~0u; }
+    __device__ __forceinline__ void early(int s, bool in) { cell = in && !d.fused ? (unsigned)d.c3_cells[s] : ~0u; }
     __device__ __forceinline__ void late() { gv = cell < nn ? g[cell] : 0.0f; }
-    __device__ __forceinline__ void done(int s, float acc) const { d.far[s] = cell < nn ? gv - acc : 0.0f; }
+    __device__ __forceinline__ void done(int s, float acc) const
+    {
+        d.far[s] = d.fused ? acc : cell < nn ? gv - acc : 0.0f;
+    }
 };
 __device__ __forceinline__ void far_wave(const SceneStep &d, int wave, int lane, GatherLds<float> &lds)
 {
@@ -295,13 +310,14 @@ __device__ __forceinline__ void far_wave(const SceneStep &d, int wave, int lane,
         wave_range(d.c3_wave, d.c3_waves, d.gran3, wave, w0, w1);
     if (d.err && *d.err)  // behind a mesh update that failed: the step is run again after the update is
         return;
-    const int t = d.st->t;
+    const int t = d.st->t + d.fused;
+    const size_t wb = window_base(d, t);
     if (wave < nw)
     {
         if (w0.x >= w1.x)
             return;
         const size_t nn = (size_t)d.a.N * d.a.N * d.a.N;
-        FarGather g{d, d.grid3 + (size_t)(((t % 3) + 3) % 3) * nn, nn, ~0u, 0.0f};
+        FarGather g{d, d.wn + wb, d.wd + wb, d.grid3 + (size_t)(((t % 3) + 3) % 3) * nn, nn, ~0u, 0.0f};
         gather_wave(g, d.c3_start, w0, w1, lane, lds);
     }
     else
@@ -312,15 +328,60 @@ __device__ __forceinline__ void far_wave(const SceneStep &d, int wave, int lane,
         {
             const float v = d.neumann[(size_t)(t - d.a.t0) * d.a.stride + i];
             d.hn[i * RING + (t & (RING - 1))] = v;
-            d.wn[i * STEPS] = v;  // tap 0 of the Dirichlet update and the near field
+            d.wn[wb + i * STEPS] = v;  // tap 0 of the Dirichlet update and the near field
         }
     }
+}
+
+// One of the eight corners a triangle's far field is interpolated from (pppm.cu:116-144): its C3
+// cell, the triangle's base cell and the interpolation weight
+struct Corner
+{
+    int ci, base;
+    float iw;
+    __device__ __forceinline__ void load(const SceneStep &d, int i)  // i = 8 * triangle + corner
+    {
+        ci = d.corner[i];  // corners of a base cell are C3 cells (>= 0)
+        iw = d.interp[i];
+        base = d.geom[i >> 3].base;
+    }
+    // g: the pressure level of the step
+    __device__ __forceinline__ float term(const SceneStep &d, const float *__restrict__ g, int w) const
+    {
+        float fv = 0.0f;
+        if (ci >= 0)
+        {
+            fv = d.far[ci];
+            if (d.fused)
+                fv = g[base + ((w >> 2) * d.a.N + (w >> 1 & 1)) * d.a.N + (w & 1)] - fv;
+        }
+        return iw * fv;
+    }
+};
+
+// The face far field of every triangle by a launch of its own, thread 8 * triangle + corner; the
+// eight terms are added in corner order
+__device__ __forceinline__ void face_far_item(const SceneStep &d, int i)
+{
+    if (i >= 8 * d.a.nt || *d.err)
+        return;  // whole groups of eight
+    const int t = d.st->t + d.fused;
+    Corner k;
+    k.load(d, i);
+    const float v = k.term(d, d.grid3 + (size_t)(((t % 3) + 3) % 3) * d.a.N * d.a.N * d.a.N, i & 7);
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 8; w++)
+        sum += __shfl(v, w, 8);
+    if ((i & 7) == 0)
+        d.ffar[i >> 3] = sum;
 }
 
 // Face far field (8-corner interpolation, pppm.cu:116-144), face near field against the
 // 4x4x4 list with D[t] = 0 and its tap-0 factors (pppm.cu:146-170), then
 // D_c[t] = (far*rc + near) / (0.5*area - sum_j D_0(c, j)) (pppm.cu:172-193).
 // The two sums of a pair are parked side by side: x the convolution, y the tap-0 factor.
+template <bool PASS>
 struct FaceGather
 {
     struct Index
@@ -328,33 +389,60 @@ struct FaceGather
         int j, rec;
     };
     const SceneStep &d;
+    const float *wn;
+    float *wd;
+    const float *g;  // pressure level of step t
     int t;
-    int s;  // this lane's segment of the chunk, -1: none
-    float ff, area;
+    int lane;
+    int s0, n;        // the group's segments s0 .. s0 + n - 1 (lane l's is s0 + l)
+    Corner k;         // corner lane & 7 of segment s0 + lane / 8
+    float ff, area;   // this lane's segment
     __device__ __forceinline__ Index load(int p) const { return Index{d.face_nbr[p], d.ofw ? p : d.face_slot[p]}; }
     __device__ __forceinline__ void conv(Index i, int n, int lane, float4 *term, float2 *vals) const
     {
-        vals[lane].x = conv_round<0, true>(d.ofw ? d.ofw : d.fw, d.ofw ? d.ofsc : d.fsc, i.rec, i.j, n, d.wn, d.wd, lane,
-                                           term, &vals[0].y);  // face_factor = (float)D_0 * scale_D
+        vals[lane].x = conv_round<0, true>(d.ofw ? d.ofw : d.fw, d.ofw ? d.ofsc : d.fsc, i.rec, i.j, n, wn, wd, lane, term,
+                                           &vals[0].y);  // face_factor = (float)D_0 * scale_D
     }
-    __device__ __forceinline__ void early(int s_, bool in) { s = in ? s_ : -1; }
+    // The face far field of the group's segments. PASS: k_face_far has left it. Else a lane per
+    // (segment, corner), eight segments at a time (a chunk of 256 pairs rarely holds more), then
+    // each segment's lane adds its eight terms in corner order.
+    __device__ __forceinline__ void early(int s, bool in)
+    {
+        s0 = __builtin_amdgcn_readfirstlane(s - lane);
+        n = (int)__popcll(__ballot(in));
+        if (!PASS && (lane >> 3) < n)
+            k.load(d, 8 * s0 + lane);
+        if (PASS && in)
+        {
+            ff = d.ffar[s];
+            area = d.geom[s].area;
+        }
+    }
     __device__ __forceinline__ void late()
     {
-        if (s < 0)
+        if (PASS)
             return;
-        int ci[8];
-        float iw[8];
-#pragma unroll
-        for (int w = 0; w < 8; w++)
-        {
-            ci[w] = d.corner[8 * s + w];  // corners of a base cell are C3 cells (>= 0)
-            iw[w] = d.interp[8 * s + w];
-        }
-        area = d.geom[s].area;
         ff = 0.0f;
+        area = 0.0f;
+        if (lane < n)
+            area = d.geom[s0 + lane].area;
+        for (int g0 = 0; g0 < n; g0 += 8)
+        {
+            float term = 0.0f;
+            if (g0 + (lane >> 3) < n)
+            {
+                if (g0 > 0)
+                    k.load(d, 8 * (s0 + g0) + lane);
+                term = k.term(d, g, lane & 7);
+            }
+            const int at = (lane - g0) & 7;
+            float sum = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 8; w++)
-            ff += iw[w] * (ci[w] >= 0 ? d.far[ci[w]] : 0.0f);
+            for (int w = 0; w < 8; w++)
+                sum += __shfl(term, 8 * at + w);
+            if (lane >= g0 && lane < g0 + 8)
+                ff = sum;
+        }
     }
     __device__ __forceinline__ void done(int s, float2 acc) const
     {
@@ -362,12 +450,13 @@ struct FaceGather
         const double den = 0.5 * (double)area - (double)acc.y;
         const float dv = (float)((double)num / den);
         d.hd[s * RING + (t & (RING - 1))] = dv;
-        d.wd[s * STEPS] = dv;  // tap 0 of the near field
+        wd[s * STEPS] = dv;  // tap 0 of the near field
     }
 };
+template <bool PASS>
 __device__ __forceinline__ void dirichlet_wave(const SceneStep &d, int wave, int lane, GatherLds<float2> &lds)
 {
-    const int t = d.st->t;
+    const int t = d.st->t + d.fused;
     if (wave >= gran_waves(d.face_waves, d.gran4))
         return;
     // the wave map is read before the error word is waited on (one memory round trip)
@@ -376,9 +465,12 @@ __device__ __forceinline__ void dirichlet_wave(const SceneStep &d, int wave, int
     // after a flagged mesh update the face lists may be incomplete: leave D[t] untouched
     if (*d.err != 0)
         return;
+    if (d.fused && wave == 0 && lane == 0)
+        d.st->next = t;
     if (w0.x >= w1.x)
         return;
-    FaceGather g{d, t, -1, 0.0f, 0.0f};
+    const size_t wb = window_base(d, t), nn = (size_t)d.a.N * d.a.N * d.a.N;
+    FaceGather<PASS> g{d, d.wn + wb, d.wd + wb, d.grid3 + (size_t)(((t % 3) + 3) % 3) * nn, t, lane, 0, 0, {}, 0.0f, 0.0f};
     gather_wave(g, d.face_start, w0, w1, lane, lds);
 }
 
@@ -390,6 +482,7 @@ struct NearGather
         int p, rec;
     };
     const SceneStep &d;
+    const float *wn, *wd;
     float *g;
     size_t nn;
     int t, lc;
@@ -398,15 +491,19 @@ struct NearGather
     __device__ __forceinline__ Index load(int p) const { return Index{p, d.c3_pairs[p]}; }
     __device__ __forceinline__ void conv(Index i, int n, int lane, float4 *term, float *vals) const
     {
-        vals[lane] = conv_round<0, false>(d.owb ? d.owb : d.wb, d.owb ? d.osb : d.sb, d.owb ? i.p : i.rec, i.rec / GC, n,
-                                          d.wn, d.wd, lane, term, nullptr);
+        vals[lane] = conv_round<0, false>(d.owb ? d.owb : d.wb, d.owb ? d.osb : d.sb, d.owb ? i.p : i.rec, i.rec / GC, n, wn,
+                                          wd, lane, term, nullptr);
     }
     __device__ __forceinline__ void early(int s, bool in)
     {
         cell = in ? (unsigned)d.c3_cells[s] : ~0u;
         fv = in ? d.far[s] : 0.0f;
     }
-    __device__ __forceinline__ void late() {}
+    __device__ __forceinline__ void late()
+    {
+        if (d.fused && cell < nn)
+            fv = g[cell] - fv;
+    }
     __device__ __forceinline__ void done(int s, float acc) const
     {
         const float v = (float)((double)fv + (double)acc * 0.98);
@@ -432,14 +529,17 @@ __device__ __forceinline__ void near_wave(const SceneStep &d, int wave, int lane
         lc = d.lc3 ? d.lc3[lane] : d.c3_index[d.lcell[lane]];
     if (d.err && *d.err)
         return;
-    const int t = d.st->t;
+    const int t = d.fused ? d.st->next : d.st->t;
+    if (d.fused && wave == 0 && lane == 0)
+        d.st->t = t;
     const size_t nn = (size_t)d.a.N * d.a.N * d.a.N;
     float *g = d.grid3 + (size_t)(((t % 3) + 3) % 3) * nn;
     if (wave < nw)
     {
         if (w0.x >= w1.x)
             return;
-        NearGather ng{d, g, nn, t, lc, ~0u, 0.0f};
+        const size_t wb = window_base(d, t);
+        NearGather ng{d, d.wn + wb, d.wd + wb, g, nn, t, lc, ~0u, 0.0f};
         gather_wave(ng, d.c3_start, w0, w1, lane, lds);
     }
     else if (d.out && wave == nw)
@@ -453,27 +553,58 @@ __device__ __forceinline__ void near_wave(const SceneStep &d, int wave, int lane
 // ---------------------------------------------------------------- single-scene kernels
 __global__ __launch_bounds__(256) void k_windows(SceneStep d, int back)
 {
-    windows_item(d, back, blockIdx.x * 256 + threadIdx.x);
+    windows_item(d, d.st->t - back + 1, blockIdx.x * 256 + threadIdx.x);
+}
+
+// The FDTD and the far-field sums of one step in one launch: the sums read only the histories, so
+// neither waits for the other. The gather's blocks come first (they run longest). A step is this
+// launch, the Dirichlet update and the near field; with the FDTD, the time advance and the far
+// field as launches of their own and the windows rebuilt in between it was five, and each costs a
+// small scene about 5 us. One pass of 64 steps alone: 32^3 1.39 -> 1.07 ms, 64^3 1.80 -> 1.50 ms.
+__global__ __launch_bounds__(TB) void k_step_head(SceneStep d, FdtdParams p, int far_blocks, int nb_inner, StatusOut f)
+{
+    static_assert(TB == BLK, "gather and FDTD blocks share the launch");
+    __shared__ GatherLds<float> lds[WPB];
+    copy_status(f);
+    if ((int)blockIdx.x < far_blocks)
+    {
+        const int wid = wave_in_block();
+        far_wave(d, xcd_wave(far_blocks >> 3, wid), threadIdx.x & 63, lds[wid]);
+        return;
+    }
+    if (*d.err)
+        return;
+    fdtd_block(d.grid3, p, d.st->t, (int)blockIdx.x - far_blocks, nb_inner);
 }
 
 __global__ __launch_bounds__(TB) void k_far(SceneStep d, int xper)
 {
     __shared__ GatherLds<float> lds[WPB];
-    const int wid = threadIdx.x >> 6;
+    const int wid = wave_in_block();
     far_wave(d, xcd_wave(xper, wid), threadIdx.x & 63, lds[wid]);
 }
 
+__global__ __launch_bounds__(256) void k_face_far(SceneStep d) { face_far_item(d, blockIdx.x * 256 + threadIdx.x); }
+
+template <bool PASS>
 __global__ __launch_bounds__(TB) void k_dirichlet(SceneStep d)
 {
     __shared__ GatherLds<float2> lds[WPB];
-    const int wid = threadIdx.x >> 6;
-    dirichlet_wave(d, blockIdx.x * WPB + wid, threadIdx.x & 63, lds[wid]);
+    const int wid = wave_in_block();
+    dirichlet_wave<PASS>(d, blockIdx.x * WPB + wid, threadIdx.x & 63, lds[wid]);
 }
 
-__global__ __launch_bounds__(TB) void k_near(SceneStep d, int xper)
+// near_blocks gather blocks, then (win2) the windows of the next step, whose ring values are all
+// written by now; they go to the half the gather does not read
+__global__ __launch_bounds__(TB) void k_near(SceneStep d, int xper, int near_blocks)
 {
     __shared__ GatherLds<float> lds[WPB];
-    const int wid = threadIdx.x >> 6;
+    if ((int)blockIdx.x >= near_blocks)
+    {
+        windows_item(d, d.st->next + 1, ((int)blockIdx.x - near_blocks) * TB + (int)threadIdx.x);
+        return;
+    }
+    const int wid = wave_in_block();
     near_wave(d, xcd_wave(xper, wid), threadIdx.x & 63, lds[wid]);
 }
 
@@ -545,55 +676,81 @@ __global__ void k_set_neumann(SceneStep d)
 }
 
 // ---------------------------------------------------------------- batched kernels
-// A batched launch covers the blocks of every scene: virtual block v belongs to scene
-// m.scene_of[v] as its local block v - m.first[scene]. Blocks go to the 8 XCDs in turn and
-// block b takes virtual block (b % 8) * m.per + b / 8, so each XCD works through one
-// contiguous run of scenes (their lists, windows and grids stay in that XCD's L2).
-__device__ __forceinline__ bool batch_block(const BatchMap &m, int &scene, int &local)
-{
-    const int v = (int)(blockIdx.x & 7) * m.per + (int)(blockIdx.x >> 3);
-    if (v >= m.total)
-        return false;
-    scene = m.scene_of[v];
-    local = v - m.first[scene];
-    return true;
-}
-
+// (map_block and scene_desc: scene_device.hpp)
 __global__ __launch_bounds__(256) void k_batch_windows(const SceneStep *__restrict__ ds, BatchMap m)
 {
     int sc, lb;
-    if (batch_block(m, sc, lb))
-        windows_item(ds[sc], 0, lb * 256 + threadIdx.x);
+    if (map_block(m, (int)blockIdx.x, sc, lb))
+        {
+        const SceneStep d = scene_desc(ds, sc);
+        windows_item(d, d.st->t + 1, lb * 256 + threadIdx.x);
+    }
+}
+
+__global__ __launch_bounds__(TB) void k_batch_head(const SceneStep *__restrict__ ds, BatchMap mf,
+                                                   const FdtdScene *__restrict__ fd, BatchMap mb)
+{
+    __shared__ GatherLds<float> lds[WPB];
+    int sc, lb;
+    if ((int)blockIdx.x < 8 * mf.per)
+    {
+        if (!map_block(mf, (int)blockIdx.x, sc, lb))
+            return;
+        const int wid = wave_in_block();
+        far_wave(scene_desc(ds, sc), lb * WPB + wid, threadIdx.x & 63, lds[wid]);
+        return;
+    }
+    if (!map_block(mb, (int)blockIdx.x - 8 * mf.per, sc, lb))
+        return;
+    const FdtdScene d = scene_desc(fd, sc);
+    fdtd_block(d.grid3, d.p, d.st->t, lb, d.nb_inner);
 }
 
 __global__ __launch_bounds__(TB) void k_batch_far(const SceneStep *__restrict__ ds, BatchMap m)
 {
     __shared__ GatherLds<float> lds[WPB];
     int sc, lb;
-    if (!batch_block(m, sc, lb))
+    if (!map_block(m, (int)blockIdx.x, sc, lb))
         return;
-    const int wid = threadIdx.x >> 6;
-    far_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, lds[wid]);
+    const int wid = wave_in_block();
+    far_wave(scene_desc(ds, sc), lb * WPB + wid, threadIdx.x & 63, lds[wid]);
 }
 
+__global__ __launch_bounds__(256) void k_batch_face_far(const SceneStep *__restrict__ ds, BatchMap m)
+{
+    int sc, lb;
+    if (map_block(m, (int)blockIdx.x, sc, lb))
+        face_far_item(scene_desc(ds, sc), lb * 256 + threadIdx.x);
+}
+
+template <bool PASS>
 __global__ __launch_bounds__(TB) void k_batch_dirichlet(const SceneStep *__restrict__ ds, BatchMap m)
 {
     __shared__ GatherLds<float2> lds[WPB];
     int sc, lb;
-    if (!batch_block(m, sc, lb))
+    if (!map_block(m, (int)blockIdx.x, sc, lb))
         return;
-    const int wid = threadIdx.x >> 6;
-    dirichlet_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, lds[wid]);
+    const int wid = wave_in_block();
+    dirichlet_wave<PASS>(scene_desc(ds, sc), lb * WPB + wid, threadIdx.x & 63, lds[wid]);
 }
 
-__global__ __launch_bounds__(TB) void k_batch_near(const SceneStep *__restrict__ ds, BatchMap m)
+__global__ __launch_bounds__(TB) void k_batch_near(const SceneStep *__restrict__ ds, BatchMap m, BatchMap mw)
 {
     __shared__ GatherLds<float> lds[WPB];
     int sc, lb;
-    if (!batch_block(m, sc, lb))
+    if ((int)blockIdx.x >= 8 * m.per)
+    {
+        if (map_block(mw, (int)blockIdx.x - 8 * m.per, sc, lb))
+        {
+            const SceneStep d = scene_desc(ds, sc);
+            windows_item(d, d.st->next + 1, lb * TB + (int)threadIdx.x);
+        }
         return;
-    const int wid = threadIdx.x >> 6;
-    near_wave(ds[sc], lb * WPB + wid, threadIdx.x & 63, lds[wid]);
+    }
+    if (!map_block(m, (int)blockIdx.x, sc, lb))
+        return;
+    const int wid = wave_in_block();
+    near_wave(scene_desc(ds, sc), lb * WPB + wid, threadIdx.x & 63, lds[wid]);
 }
 
 __global__ void k_batch_advance(const SceneStep *__restrict__ ds, int n)
@@ -626,6 +783,9 @@ int batch_blocks(const SceneStep &d, BatchKernel k)
     }
     case BatchKernel::Far:
         return blocks_for_waves(far_waves(d));
+    case BatchKernel::FaceFar:
+        return std::max(1, (int)((8LL * d.a.nt + 255) / 256));
+    case BatchKernel::DirichletOnly:
     case BatchKernel::Dirichlet:
         return blocks_for_waves(gran_waves(d.face_waves, d.gran4));
     case BatchKernel::Near:
@@ -653,14 +813,46 @@ hipError_t launch_dirichlet(const SceneStep &d, hipStream_t s)
     // plain block order: the heavy face lists of finely meshed objects sit together in the wave
     // range, and round-robin spreads them over the XCDs (the contiguous mapping of the C3 gathers
     // cut this kernel's HBM traffic from 47.6 to 39.7 MB but raised its time from 19.1 to 21.6 us)
-    k_dirichlet<<<blocks_for_waves(gran_waves(d.face_waves, d.gran4)), TB, 0, s>>>(d);
+    const int blocks = blocks_for_waves(gran_waves(d.face_waves, d.gran4));
+    if (d.ffar)
+    {
+        k_face_far<<<(8 * d.a.nt + 255) / 256, 256, 0, s>>>(d);
+        k_dirichlet<true><<<blocks, TB, 0, s>>>(d);
+    }
+    else
+        k_dirichlet<false><<<blocks, TB, 0, s>>>(d);
     return hipGetLastError();
 }
 
 hipError_t launch_near(const SceneStep &d, hipStream_t s)
 {
     const int per = xcd_per(near_waves(d));
-    k_near<<<8 * per, TB, 0, s>>>(d, per);
+    const int nwin = d.win2 ? (int)(((long long)d.a.nt * STEPS + TB - 1) / TB) : 0;
+    k_near<<<8 * per + nwin, TB, 0, s>>>(d, per, 8 * per);
+    return hipGetLastError();
+}
+
+hipError_t launch_step_head(const SceneStep &d, const FdtdParams &p, const StatusOut &status, hipStream_t s)
+{
+    int nb_inner = 0;
+    const hipError_t e = launch_fdtd_march(d.grid3, p, d.st, d.err, s, nb_inner);
+    if (e != hipSuccess)
+        return e;
+    const int far_blocks = 8 * xcd_per(far_waves(d));
+    k_step_head<<<far_blocks + nb_inner + fdtd_shell_blocks(p.N), TB, 0, s>>>(d, p, far_blocks, nb_inner, status);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_head(const SceneStep *descs, const BatchMap &mf, const FdtdScene *fd, const BatchMap &mb,
+                             hipStream_t s)
+{
+    k_batch_head<<<8 * mf.per + 8 * mb.per, TB, 0, s>>>(descs, mf, fd, mb);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_near(const SceneStep *descs, const BatchMap &mn, const BatchMap &mw, hipStream_t s)
+{
+    k_batch_near<<<8 * mn.per + 8 * mw.per, TB, 0, s>>>(descs, mn, mw);
     return hipGetLastError();
 }
 
@@ -708,11 +900,17 @@ hipError_t launch_batch(BatchKernel k, const SceneStep *descs, const BatchMap &m
     case BatchKernel::Far:
         k_batch_far<<<grid, TB, 0, s>>>(descs, m);
         break;
+    case BatchKernel::FaceFar:
+        k_batch_face_far<<<grid, 256, 0, s>>>(descs, m);
+        break;
+    case BatchKernel::DirichletOnly:
+        k_batch_dirichlet<true><<<grid, TB, 0, s>>>(descs, m);
+        break;
     case BatchKernel::Dirichlet:
-        k_batch_dirichlet<<<grid, TB, 0, s>>>(descs, m);
+        k_batch_dirichlet<false><<<grid, TB, 0, s>>>(descs, m);
         break;
     case BatchKernel::Near:
-        k_batch_near<<<grid, TB, 0, s>>>(descs, m);
+        k_batch_near<<<grid, TB, 0, s>>>(descs, m, BatchMap{});
         break;
     }
     return hipGetLastError();

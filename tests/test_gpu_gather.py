@@ -69,3 +69,47 @@ def test_entries_per_wave_agree(amd, scenes_mod, n_scenes):
         assert np.array_equal(s.get_grid(0).view(np.uint32), together[i].get_grid(0).view(np.uint32))
         for a, b in zip(s.get_history(), together[i].get_history()):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def test_step_routes_agree(amd, scenes_mod):
+    """The step in three launches, by series (windows handed from step to step) and alone, equals
+    the phase entry points and the launches of the timed step, in any order of calls."""
+    import torch
+    sc = scenes_mod.c1_static_sphere(steps=40)
+    rng = np.random.default_rng(2)
+    acc = rng.standard_normal((40, len(sc.tris))).astype(np.float32)
+    dev = torch.from_numpy(acc).cuda()
+    lis = [sc.listener, (16, 16, 23)]
+
+    def solver():
+        s = amd.PPPMSolver(sc.res, sc.dl, sc.dt, sc.min_pos, 0, 0.83, sc.c)
+        s.set_mesh(sc.verts, sc.tris)
+        return s
+
+    def phases(s, i):
+        s.fdtd_step()
+        s.solve_fdtd_far()
+        s.set_neumann_condition(acc[i])
+        s.update_dirichlet()
+        s.solve_fdtd_near()
+    a, b = solver(), solver()
+    for i in range(40):
+        phases(a, i)
+    out = torch.zeros(40, 2, device="cuda")
+    b.run(dev[:7], 7, lis, out[:7], use_graph=False)
+    b.update_grid_and_face(acc[7])
+    phases(b, 8)
+    b.run(dev[9:20], 11, lis, out[9:20], use_graph=True)
+    b.set_timing(True)
+    b.update_grid_and_face(acc[20])
+    b.run(dev[21:24], 3, lis, out[21:24], use_graph=False)
+    b.set_timing(False)
+    b.run_noalloc(dev[24:27], 3, lis, out[24:27])
+    b.update_grid_and_face(dev[27])
+    b.run(dev[28:], 12, lis, out[28:], use_graph=False)
+    assert a.time_idx() == b.time_idx()
+    for rel in (0, -1):
+        assert np.array_equal(a.get_grid(rel).view(np.uint32), b.get_grid(rel).view(np.uint32))
+    for x, y in zip(a.get_history(), b.get_history()):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+    assert np.array_equal(out[-1].cpu().numpy(), b.read_cells(lis))
