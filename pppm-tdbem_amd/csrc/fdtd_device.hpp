@@ -2,6 +2,7 @@
 // step.hip: beside the far-field gather): the leapfrog update of the interior and the first-order
 // absorbing boundary.
 #pragma once
+#include "divide.hpp"
 #include "internal.hpp"
 
 namespace pppm_amd
@@ -116,9 +117,11 @@ __device__ inline void abc_cell(float *g, const float *gm, float *gp, int N, int
 }
 
 // Leapfrog update of one interior cell from its six neighbours, in the reference's FP64
-// operation order: sum x-, x+, y-, y+, z-, z+, then -6 * centre; / h^2; 2 p + coef lap - p_prev
+// operation order: sum x-, x+, y-, y+, z-, z+, then -6 * centre; / h^2; 2 p + coef lap - p_prev.
+// rhh = uniform_rcp(p.hh), formed once per thread: an FP32-range sum over the square of an FP32
+// value stays far from FP64's exponent limits.
 __device__ __forceinline__ float leapfrog(float xm, float xp, float ym, float yp, float zm, float zp, float gc,
-                                          float gmv, const FdtdParams &p)
+                                          float gmv, const FdtdParams &p, double rhh)
 {
     double sum = 0;
     sum += xm;
@@ -128,7 +131,7 @@ __device__ __forceinline__ float leapfrog(float xm, float xp, float ym, float yp
     sum += zm;
     sum += zp;
     sum -= 6 * gc;
-    const double lap = sum / p.hh;
+    const double lap = shared_div(sum, p.hh, rhh);
     double v = 2 * gc;
     v += p.coef * lap;
     v += -gmv;
@@ -164,6 +167,7 @@ __device__ __forceinline__ void fdtd_block(float *__restrict__ grid3, const Fdtd
             const unsigned yq = q / M;
             const int y = 2 + (int)yq, z = 2 + (int)(q - yq * M), x0 = 2 + (int)xb * XC;
             const int NN2 = N * N;
+            const double rhh = uniform_rcp(p.hh);
             const int c0 = lin3(x0, y, z, N);
             float col[XC + 2], ym[XC], yp[XC], zm[XC], zp[XC], pm[XC];
 #pragma unroll
@@ -183,7 +187,7 @@ __device__ __forceinline__ void fdtd_block(float *__restrict__ grid3, const Fdtd
             for (int i = 0; i < XC; i++)
                 if (x0 + i <= N - 3)
                     // laplacian + update in FP64, sum order x-, x+, y-, y+, z-, z+, -6*centre (fdtd.cu:7-33)
-                    gp[c0 + i * NN2] = leapfrog(col[i], col[i + 2], ym[i], yp[i], zm[i], zp[i], col[i + 1], pm[i], p);
+                    gp[c0 + i * NN2] = leapfrog(col[i], col[i + 2], ym[i], yp[i], zm[i], zp[i], col[i + 1], pm[i], p, rhh);
         }
     }
     else

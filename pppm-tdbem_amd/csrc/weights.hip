@@ -15,6 +15,7 @@
 // exactly as the reference stores it. Storage: per record 16 x half2 {S_k, D_k}
 // (64 B, one half cache line) plus a float2 {scale_S, scale_D}.
 #include "detmath.hpp"
+#include "divide.hpp"
 #include "internal.hpp"
 #include "tri_device.hpp"
 
@@ -44,26 +45,10 @@ __device__ inline cdbl cexp_d(double re, double im)
     return {e * cs, e * sn};
 }
 
-// 1 / d for quotients that share the denominator d: the reciprocal estimate and two Newton steps,
-// then per quotient the product, its residual and the correction. These are the steps of the
-// compiler's own FP64 division without its range scaling, so the quotients are its bits (the
-// correctly rounded ones) as long as neither operand nor quotient comes near the exponent limits;
-// layer64_pair checks that and divides plainly otherwise.
-__device__ inline double shared_rcp(double d)
-{
-    double y = __builtin_amdgcn_rcp(d);
-    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
-    return __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
-}
-__device__ inline double shared_div(double n, double d, double y)
-{
-    const double m = n * y;
-    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d, m, n), y, m), d, n);
-}
-
 // single / double layer kernels (potential.h:22-47) of one (source point, target) pair, split in
 // two: the part without the wave number, computed once for the 9 wave numbers (r = |trg - src|,
-// the denominators 4 pi r and 4 pi r^2 r with their shared reciprocals, and (src - trg) . n),
+// the denominators 4 pi r and 4 pi r^2 r with their shared reciprocals (layer64_pair checks that no
+// operand or quotient comes near the exponent limits and divides plainly otherwise), and (src - trg) . n),
 // and the part per wave number, whose complex exponential serves both layers. r = 0: the target
 // is the source point and both kernels are 0. y0 = 0: the denominators are divided by plainly.
 struct LayerTarget
