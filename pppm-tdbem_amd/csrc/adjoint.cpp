@@ -251,6 +251,22 @@ size_t state_bytes(const pppm_solver *s)
     return 2 * NN * sizeof(float) + 2 * (size_t)s->nt * RING * sizeof(float) + 16;
 }
 
+// a saved state that a kernel can read and write as words: 4-byte aligned, in this device's memory
+// (host memory, another device's and odd addresses take copies)
+bool words_here(const void *p)
+{
+    hipPointerAttribute_t a{};
+    int dev = -1;
+    if ((uintptr_t)p % 4 || hipGetDevice(&dev) != hipSuccess)
+        return false;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == dev;
+}
+
 float *level_ptr(pppm_solver *s, int t, int rel)
 {
     const size_t NN = (size_t)s->N * s->N * s->N;
@@ -308,11 +324,15 @@ int pppm_adjoint_reset(pppm_solver *s, int t_last)
         return solver_fail(s, PPPM_ERR_ARG, "adjoint: grid edges from 8 and grids below 2^31 cells");
     ARC(adjoint_setup(s));
     const size_t NN = (size_t)s->N * s->N * s->N;
-    ACK(hipMemsetAsync(s->adj_lam3.p, 0, 3 * NN * sizeof(float), s->stream));
-    ACK(hipMemsetAsync(s->adj_ln.p, 0, (size_t)s->nt * RING * sizeof(float), s->stream));
-    ACK(hipMemsetAsync(s->adj_ld.p, 0, (size_t)s->nt * RING * sizeof(float), s->stream));
-    AdjState st{t_last, 0};
-    ACK(hipMemcpyAsync(s->adj_state.p, &st, sizeof(st), hipMemcpyHostToDevice, s->stream));
+    static_assert(sizeof(AdjState) == 2 * sizeof(int), "AdjState is {t, pad}");
+    WordRanges r{};
+    r.add(s->adj_lam3.p, nullptr, 3 * NN);
+    r.add(s->adj_ln.p, nullptr, (size_t)s->nt * RING);
+    r.add(s->adj_ld.p, nullptr, (size_t)s->nt * RING);
+    r.ints = reinterpret_cast<int *>(s->adj_state.p);
+    r.n_ints = 2;
+    r.v[0] = t_last;
+    ACK(launch_word_ranges(r, s->stream));
     ACK(hipStreamSynchronize(s->stream));
     s->adj_t = t_last;
     return PPPM_OK;
@@ -387,11 +407,24 @@ int pppm_save_state(pppm_solver *s, void *dst_dev)
     const size_t NN = (size_t)s->N * s->N * s->N, R = (size_t)s->nt * RING;
     unsigned char *p = (unsigned char *)dst_dev;
     const int t = s->t_host;
-    ACK(hipMemcpyAsync(p, level_ptr(s, t, 0), NN * 4, hipMemcpyDeviceToDevice, s->stream));
-    ACK(hipMemcpyAsync(p + NN * 4, level_ptr(s, t, -1), NN * 4, hipMemcpyDeviceToDevice, s->stream));
-    ACK(hipMemcpyAsync(p + 2 * NN * 4, s->hn.p, R * 4, hipMemcpyDeviceToDevice, s->stream));
-    ACK(hipMemcpyAsync(p + 2 * NN * 4 + R * 4, s->hd.p, R * 4, hipMemcpyDeviceToDevice, s->stream));
-    ACK(launch_put_ints(reinterpret_cast<int *>(p + 2 * NN * 4 + 2 * R * 4), 4, t, s->N, s->nt, 0x5157, s->stream));
+    if (!words_here(p))
+    {
+        ACK(hipMemcpyAsync(p, level_ptr(s, t, 0), NN * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(hipMemcpyAsync(p + NN * 4, level_ptr(s, t, -1), NN * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(hipMemcpyAsync(p + 2 * NN * 4, s->hn.p, R * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(hipMemcpyAsync(p + 2 * NN * 4 + R * 4, s->hd.p, R * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(launch_put_ints(reinterpret_cast<int *>(p + 2 * NN * 4 + 2 * R * 4), 4, t, s->N, s->nt, 0x5157, s->stream));
+        return PPPM_OK;
+    }
+    WordRanges r{};
+    r.add(p, level_ptr(s, t, 0), NN);
+    r.add(p + NN * 4, level_ptr(s, t, -1), NN);
+    r.add(p + 2 * NN * 4, s->hn.p, R);
+    r.add(p + 2 * NN * 4 + R * 4, s->hd.p, R);
+    r.ints = reinterpret_cast<int *>(p + 2 * NN * 4 + 2 * R * 4);
+    r.n_ints = 4;
+    r.v[0] = t, r.v[1] = s->N, r.v[2] = s->nt, r.v[3] = 0x5157;
+    ACK(launch_word_ranges(r, s->stream));
     return PPPM_OK;
 }
 
@@ -409,11 +442,25 @@ int pppm_load_state(pppm_solver *s, const void *src_dev)
     if (trailer[3] != 0x5157 || trailer[1] != s->N || trailer[2] != s->nt || trailer[0] < -1)
         return solver_fail(s, PPPM_ERR_ARG, "load_state: not a state of this solver's grid and mesh");
     const int t = trailer[0];
-    ACK(hipMemcpyAsync(level_ptr(s, t, 0), p, NN * 4, hipMemcpyDeviceToDevice, s->stream));
-    ACK(hipMemcpyAsync(level_ptr(s, t, -1), p + NN * 4, NN * 4, hipMemcpyDeviceToDevice, s->stream));
-    ACK(hipMemcpyAsync(s->hn.p, p + 2 * NN * 4, R * 4, hipMemcpyDeviceToDevice, s->stream));
-    ACK(hipMemcpyAsync(s->hd.p, p + 2 * NN * 4 + R * 4, R * 4, hipMemcpyDeviceToDevice, s->stream));
-    return pppm_set_time_idx(s, t);
+    if (!words_here(p))
+    {
+        ACK(hipMemcpyAsync(level_ptr(s, t, 0), p, NN * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(hipMemcpyAsync(level_ptr(s, t, -1), p + NN * 4, NN * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(hipMemcpyAsync(s->hn.p, p + 2 * NN * 4, R * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(hipMemcpyAsync(s->hd.p, p + 2 * NN * 4 + R * 4, R * 4, hipMemcpyDeviceToDevice, s->stream));
+        return pppm_set_time_idx(s, t);
+    }
+    WordRanges r{};
+    r.add(level_ptr(s, t, 0), p, NN);
+    r.add(level_ptr(s, t, -1), p + NN * 4, NN);
+    r.add(s->hn.p, p + 2 * NN * 4, R);
+    r.add(s->hd.p, p + 2 * NN * 4 + R * 4, R);
+    r.ints = reinterpret_cast<int *>(s->state.p);
+    r.n_ints = 2;
+    r.v[0] = t;
+    ACK(launch_word_ranges(r, s->stream));
+    s->t_host = t;
+    return PPPM_OK;
 }
 
 }  // extern "C"

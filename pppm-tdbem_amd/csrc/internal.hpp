@@ -126,6 +126,25 @@ hipError_t launch_fill_int(int *a, long long n, int value, hipStream_t s);
 // a[0..n) = v[0..n) for n <= 4, from the launch arguments: a stream-ordered small write that
 // needs no host buffer to outlive the call (so no wait for the stream)
 hipError_t launch_put_ints(int *a, int n, int v0, int v1, int v2, int v3, hipStream_t s);
+// Up to four ranges of 4-byte words copied (src null: cleared) and up to four ints written, in one
+// launch; addresses are multiples of 4, ranges of one set do not overlap
+struct WordRanges
+{
+    static constexpr int MAX = 4;
+    unsigned *dst[MAX];
+    const unsigned *src[MAX];
+    long long words[MAX];
+    int n;
+    int *ints;
+    int n_ints, v[4];
+    void add(void *d, const void *s_, size_t w)
+    {
+        dst[n] = static_cast<unsigned *>(d);
+        src[n] = static_cast<const unsigned *>(s_);
+        words[n++] = (long long)w;
+    }
+};
+hipError_t launch_word_ranges(const WordRanges &r, hipStream_t s);
 hipError_t launch_copy_verts(const float *series, long long stride, int t0, const StepState *st, float *verts, int n,
                              hipStream_t s);
 // per-tile counts of the dirty face pairs, accumulated by the face lookup for the face-pair scan

@@ -1498,16 +1498,20 @@ int pppm_reset(pppm_solver *s)
     if (check_handle(s))
         return PPPM_ERR_ARG;
     const size_t NN = (size_t)s->N * s->N * s->N;
-    CK(hipMemsetAsync(s->grid.p, 0, 3 * NN * sizeof(float), s->stream));
+    static_assert(sizeof(StepState) == 2 * sizeof(int), "StepState is {t, next}");
+    WordRanges r{};
+    r.add(s->grid.p, nullptr, 3 * NN);
     if (s->use_pml)
-        CK(hipMemsetAsync(s->pmlbuf.p, 0, 3 * NN * 6 * sizeof(float), s->stream));
+        r.add(s->pmlbuf.p, nullptr, 3 * NN * 6);
     if (s->mesh_set)
     {
-        CK(hipMemsetAsync(s->hn.p, 0, (size_t)s->nt * RING * sizeof(float), s->stream));
-        CK(hipMemsetAsync(s->hd.p, 0, (size_t)s->nt * RING * sizeof(float), s->stream));
+        r.add(s->hn.p, nullptr, (size_t)s->nt * RING);
+        r.add(s->hd.p, nullptr, (size_t)s->nt * RING);
     }
-    static_assert(sizeof(StepState) == 2 * sizeof(int), "StepState is {t, next}");
-    CK(launch_put_ints(reinterpret_cast<int *>(s->state.p), 2, -1, 0, 0, 0, s->stream));
+    r.ints = reinterpret_cast<int *>(s->state.p);
+    r.n_ints = 2;
+    r.v[0] = -1;
+    CK(launch_word_ranges(r, s->stream));
     s->t_host = -1;
     return PPPM_OK;
 }
