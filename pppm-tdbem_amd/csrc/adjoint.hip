@@ -28,6 +28,8 @@
 #include "scene_device.hpp"
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 namespace pppm_amd
 {
@@ -74,9 +76,29 @@ __device__ __forceinline__ void adj_read(const AdjScene &d, int blk)
     }
 }
 
+// body(integral_constant<int, 0>) .. body(integral_constant<int, N - 1>), in order
+template <class F, int... M>
+__device__ __forceinline__ void unrolled_seq(F &&body, std::integer_sequence<int, M...>)
+{
+    (body(std::integral_constant<int, M>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void unrolled(F &&body)
+{
+    unrolled_seq(body, std::make_integer_sequence<int, N>{});
+}
+// lane M's value of each aligned 16-lane group, by a row broadcast in the vector unit (a shuffle
+// goes through LDS)
+template <int M>
+__device__ __forceinline__ float group_bcast(float x)
+{
+    const int v = __float_as_int(x);
+    return __int_as_float(__builtin_amdgcn_update_dpp(v, v, 0x150 + M, 0xf, 0xf, false));
+}
+
 // The 16 tap threads of a triangle are one aligned 16-lane group (a block's first thread is at
 // a multiple of 16 within its triangle range); lane k fetches the per-record values of records
-// k and k + 16 of the triangle's 27, and every lane takes record o's from lane o % 16 by shuffle.
+// k and k + 16 of the triangle's 27, and every lane takes record o's from lane o % 16 by a row broadcast.
 struct RecVals
 {
     float v[2];
@@ -101,12 +123,13 @@ __device__ __forceinline__ RecVals rec_vals(const int *__restrict__ tc3, const f
     }
     return r;
 }
-__device__ __forceinline__ void rec_take(const RecVals &r, int o, float &v, float2 &sc)
+template <int O>
+__device__ __forceinline__ void rec_take(const RecVals &r, float &v, float2 &sc)
 {
-    const int h = o / STEPS, src = o % STEPS;
-    v = __shfl(r.v[h], src, STEPS);
-    sc.x = __shfl(r.sc[h].x, src, STEPS);
-    sc.y = __shfl(r.sc[h].y, src, STEPS);
+    constexpr int h = O / STEPS, src = O % STEPS;
+    v = group_bcast<src>(r.v[h]);
+    sc.x = group_bcast<src>(r.sc[h].x);
+    sc.y = group_bcast<src>(r.sc[h].y);
 }
 
 // 2. near field transposed, one thread per (triangle, tap): the 27 records of a triangle are
@@ -120,17 +143,15 @@ __device__ __forceinline__ void adj_near(const AdjScene &d, int blk)
     const int tri = i / STEPS, k = i % STEPS;
     const RecVals rv = rec_vals(d.tc3, d.unear, d.sb, tri, k);
     float an = 0.0f, ad = 0.0f;
-#pragma unroll
-    for (int o = 0; o < GC; o++)
-    {
+    unrolled<GC>([&](auto o) {
         const int rec = tri * GC + o;
         float u;
         float2 sc;
-        rec_take(rv, o, u, sc);
+        rec_take<o>(rv, u, sc);
         const uint32_t w = d.wb[(size_t)rec * STEPS + k];
         an += wS(w, sc) * u;
         ad += wD(w, sc) * u;
-    }
+    });
     const int slot = tri * RING + ((t - k) & (RING - 1));
     d.ln[slot] += -0.98f * an;
     d.ld[slot] += 0.98f * ad;
@@ -154,7 +175,8 @@ __device__ __forceinline__ int c3_part_blocks(const AdjScene &d) { return (d.n_c
 // 4. Dirichlet transposed: C3 cells [0, n_c3) gather the face-far-field interpolation; then one
 // thread per (triangle j, tap) gathers the face pairs (c, j) (records in that order: a
 // triangle's 16 lanes read consecutive 64 B records; lane k fetches pair eb + k's cell value and
-// scales, shared by shuffles)
+// scales, handed on by row broadcasts). Bound by the latency of the record stream: 82k triangles with
+// 128 pairs each, one record load in flight and LDS shuffles 403 us; 16 loads first 240 us
 __device__ __forceinline__ void adj_dir(const AdjScene &d, int blk)
 {
     const int t = d.ast->t;
@@ -177,26 +199,29 @@ __device__ __forceinline__ void adj_dir(const AdjScene &d, int blk)
     const int j = q / STEPS, k = q % STEPS;
     const int e0 = d.ft_start[j], e1 = d.ft_start[j + 1];
     float an = 0.0f, ad = 0.0f;
-    for (int eb = e0; eb < e1; eb += STEPS)
-    {
-        const int el = eb + k;
-        float vl = 0.0f;
-        float2 sl = make_float2(0.0f, 0.0f);
-        if (el < e1)
-        {
-            vl = d.v[d.ft_c[el]];
-            sl = d.tfsc[el];
-        }
-        const int n = min(STEPS, e1 - eb);
-        for (int m = 0; m < n; m++)
-        {
-            const float vc = __shfl(vl, m, STEPS);
-            const float2 sc = make_float2(__shfl(sl.x, m, STEPS), __shfl(sl.y, m, STEPS));
-            const uint32_t w = d.tfw[(size_t)(eb + m) * STEPS + k];
-            an += wS(w, sc) * vc;
-            ad += wD(w, sc) * vc;
-        }
-    }
+    // a run of 16 pairs: their records' loads first, then the sums in pair order; lanes past a last
+    // short run load its last pair (not added)
+    auto run = [&](int eb, auto is_full) {
+        constexpr bool full = decltype(is_full)::value;
+        const int last = full ? eb + STEPS - 1 : e1 - 1;
+        const int el = min(eb + k, last);
+        const float vl = d.v[d.ft_c[el]];
+        const float2 sl = d.tfsc[el];
+        uint32_t w[STEPS];
+        unrolled<STEPS>([&](auto m) { w[m] = d.tfw[(size_t)min(eb + m, last) * STEPS + k]; });
+        unrolled<STEPS>([&](auto m) {
+            const float vc = group_bcast<m>(vl);
+            const float2 sc = make_float2(group_bcast<m>(sl.x), group_bcast<m>(sl.y));
+            const float pn = an + wS(w[m], sc) * vc, pd = ad + wD(w[m], sc) * vc;
+            if (full || eb + m <= last)
+                an = pn, ad = pd;
+        });
+    };
+    int eb = e0;
+    for (; eb + STEPS <= e1; eb += STEPS)
+        run(eb, std::true_type{});
+    if (eb < e1)
+        run(eb, std::false_type{});
     const int rs = j * RING + ((t - k) & (RING - 1));
     d.ln[rs] += -an;
     if (k > 0)  // D_j[t] enters the face near field as 0 (pppm.cu:143)
@@ -226,17 +251,15 @@ __device__ __forceinline__ void adj_far(const AdjScene &d, int blk)
     // every lane of the group takes part in the shuffles; tap 0 then writes the gradient instead
     const RecVals rv = rec_vals(d.tc3, d.lfar, d.sf, tri, k);
     float an = 0.0f, ad = 0.0f;
-#pragma unroll
-    for (int o = 0; o < GC; o++)
-    {
+    unrolled<GC>([&](auto o) {
         const int rec = tri * GC + o;
         float lf;
         float2 sc;
-        rec_take(rv, o, lf, sc);
+        rec_take<o>(rv, lf, sc);
         const uint32_t w = d.wf[(size_t)rec * STEPS + k];
         an += wS(w, sc) * lf;
         ad += wD(w, sc) * lf;
-    }
+    });
     if (k == 0)
     {
         const int slot = tri * RING + (t & (RING - 1));
