@@ -29,7 +29,8 @@ __device__ __forceinline__ T const_load(const T *p)
 template <class T>
 __device__ __forceinline__ void as_global(T *&p)
 {
-    p = (T *)(__attribute__((address_space(1))) T *)p;
+    // by way of an integer: a cast to global and back would be folded away
+    p = (T *)(__attribute__((address_space(1))) T *)(unsigned long long)p;
 }
 template <class... P>
 __device__ __forceinline__ void all_global(P &...p)
