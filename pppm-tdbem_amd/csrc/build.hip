@@ -403,6 +403,33 @@ hipError_t launch_put_ints(int *a, int n, int v0, int v1, int v2, int v3, hipStr
     k_put_ints<<<1, WAVE, 0, s>>>(a, n, v0, v1, v2, v3);
     return hipGetLastError();
 }
+// Thread v: the last scene whose first virtual block is at or before v (empty scenes share their
+// successor's first block), by bisection; the threads also copy the firsts.
+__global__ __launch_bounds__(B) void k_scene_map(const int *__restrict__ first, int n, int total,
+                                                 int *__restrict__ first_out, int *__restrict__ scene_of)
+{
+    const int v = blockIdx.x * B + threadIdx.x;
+    if (v < n)
+        first_out[v] = first[v];
+    if (v >= total)
+        return;
+    int lo = 0, hi = n;  // first[lo] <= v < first[hi]
+    while (hi - lo > 1)
+    {
+        const int m = (lo + hi) >> 1;
+        if (first[m] <= v)
+            lo = m;
+        else
+            hi = m;
+    }
+    scene_of[v] = lo;
+}
+hipError_t launch_scene_map(const int *first, int n, int total, int *first_out, int *scene_of, hipStream_t s)
+{
+    k_scene_map<<<nblk(std::max(n, total)), B, 0, s>>>(first, n, total, first_out, scene_of);
+    return hipGetLastError();
+}
+
 // Blocks [first[k], first[k + 1]) take range k, RW words each, a thread four 16-byte accesses one
 // block width apart where both addresses allow them, else sixteen of 4 bytes. Bound by memory, or for
 // a small state by its launch: a reset was five launches (fills and the time index), 15 us of a

@@ -430,6 +430,8 @@ struct BatchMap
     const int *first;
     int total, per;
 };
+// first_out = first (n scenes) and scene_of[v] = the scene of virtual block v < total
+hipError_t launch_scene_map(const int *first, int n, int total, int *first_out, int *scene_of, hipStream_t s);
 enum class BatchKernel
 {
     Windows,
