@@ -248,7 +248,7 @@ __device__ __forceinline__ void adj_far(const AdjScene &d, int blk)
     if (q >= d.nt * STEPS)
         return;  // whole 16-lane groups
     const int tri = q / STEPS, k = q % STEPS;
-    // every lane of the group takes part in the shuffles; tap 0 then writes the gradient instead
+    // every lane of the group takes part in the broadcasts; tap 0 then writes the gradient instead
     const RecVals rv = rec_vals(d.tc3, d.lfar, d.sf, tri, k);
     float an = 0.0f, ad = 0.0f;
     unrolled<GC>([&](auto o) {

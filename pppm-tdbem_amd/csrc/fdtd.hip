@@ -38,11 +38,12 @@ constexpr int kMarchMin = 128;
 // of this plane's store.
 //
 // STREAM: the previous level is read and the next one written past the caches, which leaves them
-// to the level-t rows that several waves read. It pays once the three levels do not fit the
-// Infinity Cache, where the next step would find them otherwise: 512^3 384 -> 367 us a step
-// (1.61 GB, 4.4 TB/s; a copy reaches 4.8), but 141^3 29 -> 37 us, so smaller grids keep to plain
-// accesses. The division by h^2 takes the reciprocal from scalar registers (141^3: 30 -> 29 us).
-constexpr long long kStreamBytes = 256LL << 20;
+// to the level-t rows that several waves read. It pays where two of the three levels no longer fit
+// the Infinity Cache (256 MB), so that the next step would not find them there: a step at 512^3
+// 384 -> 367 us (1.61 GB, 4.4 TB/s; a copy reaches 4.8), with the shell 448^3 365 -> 344 and
+// 352^3 214 -> 195 us, but 284^3 140 -> 175 and 141^3 29 -> 37 us; at 316^3 it gives nothing. The
+// division by h^2 takes the reciprocal from scalar registers (141^3: 30 -> 29 us).
+constexpr long long kStreamBytes = 384LL << 20;  // of three levels
 constexpr int MTY = 16;
 constexpr int MBLK = 64 * MTY;
 constexpr int MCPT = 4;            // z columns per thread, 64 apart: a tile is 16 rows x 256 z

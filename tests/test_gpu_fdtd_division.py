@@ -49,7 +49,7 @@ def test_division_bitexact(amd, oracle_mod, n, h, kind):
     assert _same(a, b)
 
 
-@pytest.mark.parametrize("n", [281, 282])  # three levels just below and just above 256 MB
+@pytest.mark.parametrize("n", [322, 323])  # three levels just below and just above 384 MB
 def test_stream_rule_bitexact(amd, oracle_mod, n):
     rng = np.random.default_rng(n)
     a, b = _levels(amd, oracle_mod, n, 0.01, lambda shape: rng.standard_normal(shape, dtype=np.float32), 2)
