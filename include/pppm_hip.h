@@ -161,7 +161,8 @@ int pppm_batch_get_timing(pppm_batch *b, double *ms8, long long *count8);
  *   handle's stream, as pppm_run.
  * pppm_state_bytes / pppm_save_state / pppm_load_state: a checkpoint of the forward state
  *   (grid levels t and t-1 with the ghost layer, both history rings, t) in caller-owned device
- *   memory; loading one restores the solver to that step (same grid and mesh only). */
+ *   memory of pppm_state_bytes bytes (saving: PPPM_ERR_HIP if its allocation ends before that);
+ *   loading one restores the solver to that step (same grid and mesh only). */
 int pppm_adjoint_reset(pppm_solver *s, int t_last);
 int pppm_adjoint_run(pppm_solver *s, const float *gout_dev, int steps, const int *listen_xyz, int n_listen,
                      float *grad_dev, long long grad_stride, int use_graph);

@@ -251,11 +251,28 @@ size_t state_bytes(const pppm_solver *s)
     return 2 * NN * sizeof(float) + 2 * (size_t)s->nt * RING * sizeof(float) + 16;
 }
 
-// a saved state that a kernel can read and write as words: 4-byte aligned, in this device's memory
-// (host memory, another device's and odd addresses take copies)
-bool words_here(const void *p)
+// bytes from p to the end of its allocation; false if p is in none that the runtime knows
+bool bytes_left(const void *p, size_t &left)
+{
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, const_cast<void *>(p)) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    const size_t off = (size_t)((uintptr_t)p - (uintptr_t)base);
+    left = off <= size ? size - off : 0;
+    return true;
+}
+
+// a saved state of `bytes` that a kernel can read and write as words: 4-byte aligned and whole inside
+// one allocation of this device (host memory, another device's, odd addresses and buffers too small
+// take copies, whose ranges the runtime checks: it refuses one that leaves its allocation)
+bool words_here(const void *p, size_t bytes)
 {
     hipPointerAttribute_t a{};
+    size_t left = 0;
     int dev = -1;
     if ((uintptr_t)p % 4 || hipGetDevice(&dev) != hipSuccess)
         return false;
@@ -264,7 +281,17 @@ bool words_here(const void *p)
         (void)hipGetLastError();
         return false;
     }
-    return a.type == hipMemoryTypeDevice && a.device == dev;
+    return a.type == hipMemoryTypeDevice && a.device == dev && bytes_left(p, left) && bytes <= left;
+}
+
+// a copy on the device; the error of one that the runtime refuses is returned here and not kept for
+// the check of a later launch
+hipError_t copy_range(void *dst, const void *src, size_t bytes, hipStream_t stream)
+{
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, stream);
+    if (e != hipSuccess)
+        (void)hipGetLastError();
+    return e;
 }
 
 float *level_ptr(pppm_solver *s, int t, int rel)
@@ -407,12 +434,16 @@ int pppm_save_state(pppm_solver *s, void *dst_dev)
     const size_t NN = (size_t)s->N * s->N * s->N, R = (size_t)s->nt * RING;
     unsigned char *p = (unsigned char *)dst_dev;
     const int t = s->t_host;
-    if (!words_here(p))
+    if (!words_here(p, state_bytes(s)))
     {
-        ACK(hipMemcpyAsync(p, level_ptr(s, t, 0), NN * 4, hipMemcpyDeviceToDevice, s->stream));
-        ACK(hipMemcpyAsync(p + NN * 4, level_ptr(s, t, -1), NN * 4, hipMemcpyDeviceToDevice, s->stream));
-        ACK(hipMemcpyAsync(p + 2 * NN * 4, s->hn.p, R * 4, hipMemcpyDeviceToDevice, s->stream));
-        ACK(hipMemcpyAsync(p + 2 * NN * 4 + R * 4, s->hd.p, R * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(copy_range(p, level_ptr(s, t, 0), NN * 4, s->stream));
+        ACK(copy_range(p + NN * 4, level_ptr(s, t, -1), NN * 4, s->stream));
+        ACK(copy_range(p + 2 * NN * 4, s->hn.p, R * 4, s->stream));
+        ACK(copy_range(p + 2 * NN * 4 + R * 4, s->hd.p, R * 4, s->stream));
+        // the trailer comes from a kernel: looked for from the ring's last word, which has been copied
+        size_t left = 0;
+        if (bytes_left(p + 2 * NN * 4 + 2 * R * 4 - 4, left) && left < 4 + 16)
+            return solver_fail(s, PPPM_ERR_HIP, "save_state: the buffer is smaller than the state");
         ACK(launch_put_ints(reinterpret_cast<int *>(p + 2 * NN * 4 + 2 * R * 4), 4, t, s->N, s->nt, 0x5157, s->stream));
         return PPPM_OK;
     }
@@ -442,12 +473,12 @@ int pppm_load_state(pppm_solver *s, const void *src_dev)
     if (trailer[3] != 0x5157 || trailer[1] != s->N || trailer[2] != s->nt || trailer[0] < -1)
         return solver_fail(s, PPPM_ERR_ARG, "load_state: not a state of this solver's grid and mesh");
     const int t = trailer[0];
-    if (!words_here(p))
+    if (!words_here(p, state_bytes(s)))
     {
-        ACK(hipMemcpyAsync(level_ptr(s, t, 0), p, NN * 4, hipMemcpyDeviceToDevice, s->stream));
-        ACK(hipMemcpyAsync(level_ptr(s, t, -1), p + NN * 4, NN * 4, hipMemcpyDeviceToDevice, s->stream));
-        ACK(hipMemcpyAsync(s->hn.p, p + 2 * NN * 4, R * 4, hipMemcpyDeviceToDevice, s->stream));
-        ACK(hipMemcpyAsync(s->hd.p, p + 2 * NN * 4 + R * 4, R * 4, hipMemcpyDeviceToDevice, s->stream));
+        ACK(copy_range(level_ptr(s, t, 0), p, NN * 4, s->stream));
+        ACK(copy_range(level_ptr(s, t, -1), p + NN * 4, NN * 4, s->stream));
+        ACK(copy_range(s->hn.p, p + 2 * NN * 4, R * 4, s->stream));
+        ACK(copy_range(s->hd.p, p + 2 * NN * 4 + R * 4, R * 4, s->stream));
         return pppm_set_time_idx(s, t);
     }
     WordRanges r{};

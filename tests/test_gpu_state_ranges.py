@@ -49,3 +49,57 @@ def test_state_round_trip(amd, n, nt, offset):
     assert torch.equal(out, out2)
     a.reset()
     assert a.time_idx() == -1 and all(not x.any() for x in _state(a))
+
+
+@pytest.mark.parametrize("missing", [0, 4, 16, 80, 300])
+def test_buffer_too_small_is_refused(amd, missing):
+    """A buffer that ends before the state does (by less than its allocation's last page holds) is
+    refused through the C ABI, which has only the pointer; one of exactly the state's size is not."""
+    import ctypes
+    import torch
+    torch.cuda.init()
+    a = _solver(amd, 20, 3)
+    a.run(torch.ones(2, 3, device="cuda"), 2, [(10, 10, 10)], torch.zeros(2, 1, device="cuda"))
+    torch.cuda.synchronize()
+    size = a.state_bytes()
+    assert -size % 4096 >= 16 and missing < size % 4096  # past the buffer is still the same page
+    p = ctypes.c_void_p()  # (the library's handle also finds the HIP runtime it is linked to)
+    assert a.lib.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size - missing)) == 0
+    try:
+        rc = a.lib.pppm_save_state(a.h, p)
+        assert (rc != 0) == (missing > 0)
+        a.save_state(torch.empty(size, dtype=torch.uint8, device="cuda"))  # the refusal leaves no error behind
+        if not missing:
+            want = _state(a)
+            a.reset()
+            assert a.lib.pppm_load_state(a.h, p) == 0 and a.time_idx() == 1
+            for x, y in zip(_state(a), want):
+                assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+        torch.cuda.synchronize()
+    finally:
+        assert a.lib.hipFree(p) == 0
+
+
+def test_save_state_is_captured(amd):
+    """save_state in a caller's graph, replayed, with steps of the caller's own between the replays."""
+    import torch
+    a = _solver(amd, 23, 5)
+    side = torch.cuda.Stream()
+    a.set_stream(side.cuda_stream)
+    size = a.state_bytes()
+    buf, want = (torch.zeros(size, dtype=torch.uint8, device="cuda") for _ in range(2))
+    acc, out = torch.ones(3, 5, device="cuda"), torch.zeros(3, 1, device="cuda")
+    torch.cuda.synchronize()
+    a.run(acc, 3, [(11, 11, 11)], out)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        a.save_state(buf)
+    for _ in range(3):  # three steps move the levels round to where they were captured
+        torch.cuda.synchronize()
+        a.run(acc, 3, [(11, 11, 11)], out)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        a.save_state(want)
+        torch.cuda.synchronize()
+        assert torch.equal(buf[:size - 16], want[:size - 16])  # the time index is the captured one
