@@ -47,10 +47,17 @@ __device__ inline cdbl cexp_d(double re, double im)
 
 // single / double layer kernels (potential.h:22-47) of one (source point, target) pair, split in
 // two: the part without the wave number, computed once for the 9 wave numbers (r = |trg - src|,
-// the denominators 4 pi r and 4 pi r^2 r with their shared reciprocals (layer64_pair checks that no
-// operand or quotient comes near the exponent limits and divides plainly otherwise), and (src - trg) . n),
+// the denominators 4 pi r and 4 pi r^2 r with their shared reciprocals, and (src - trg) . n),
 // and the part per wave number, whose complex exponential serves both layers. r = 0: the target
 // is the source point and both kernels are 0. y0 = 0: the denominators are divided by plainly.
+//
+// The shared reciprocals are taken for R_MIN < r < R_MAX and exponents |Re z| < Z_MAX, where no step of
+// the division comes near the exponent limits: the denominators lie between 2^-147 and 2^52, |e^z|
+// between 2^-866 and 2^866 and its parts above 2^-930 (a sine or cosine of a double below 2^20 is 0
+// or above 2^-60), so the quotients lie between 2^-982 and 2^1013, and a remainder, 105 bits below its
+// numerator, is a whole number of the smallest subnormals. Grids have r of their cell sizes (1e-3 to
+// 1 m) and far from either end.
+constexpr double R_MIN = 0x1p-50, R_MAX = 0x1p16, Z_MAX = 600.0;
 struct LayerTarget
 {
     double r, q0, y0, q1, y1, dn;
@@ -64,7 +71,7 @@ __device__ inline LayerTarget layer_target(d3 src, d3 trg, d3 n)
     const double r = sqrt(r2);
     const d3 s1 = src - trg;  // = -s0 exactly, so dotd(s1, s1) == r2
     const double q0 = 4 * PI_R * r, q1 = 4 * PI_R * r2 * r;
-    const bool plain = !(r > 1e-60 && r < 1e60);
+    const bool plain = !(r > R_MIN && r < R_MAX);
     return {r, q0, plain ? 0.0 : shared_rcp(q0), q1, plain ? 0.0 : shared_rcp(q1), dotd(s1, n)};
 }
 // e^(x + i y) for |x| < 600 and |y| < 2^19: det_exp and det_sincos (detmath.hpp) without their
@@ -104,7 +111,7 @@ __device__ inline void layer64_pair(const LayerTarget &t, double kr, double ki, 
 {
     const double zr = -t.r * ki, zi = t.r * kr;
     double ar, ai;
-    if (t.y0 != 0 && fabs(zr) < 600.0 && fabs(zi) < 5e5)  // |e^z| and its parts stay above 2^-930
+    if (t.y0 != 0 && fabs(zr) < Z_MAX && fabs(zi) < 5e5)
     {
         const cdbl e = cexp_mid(zr, zi);
         g0 = {shared_div(e.re, t.q0, t.y0), shared_div(e.im, t.q0, t.y0)};

@@ -32,14 +32,26 @@ def _mesh(name):
 @pytest.mark.parametrize("name", ["soup1", "soup2", "soup3", "soup8", "soup23", "corner", "edge", "duplicate",
                                   "coincident", "sphere"])
 def test_weights_bitexact(amd, oracle_mod, scenes_mod, name, dt_scale):
+    _compare(amd, oracle_mod, scenes_mod, name, dt_scale, 1.0)
+
+
+# cells of 1e-15 and 2e4: distances on both sides of either end of the shared reciprocals' range
+@pytest.mark.parametrize("scale", [1e-13, 2e6])
+@pytest.mark.parametrize("name", ["soup8", "duplicate", "sphere"])
+def test_weights_bitexact_at_scale(amd, oracle_mod, scenes_mod, name, scale):
+    _compare(amd, oracle_mod, scenes_mod, name, 1.0, scale)
+
+
+def _compare(amd, oracle_mod, scenes_mod, name, dt_scale, scale):
     if name == "sphere":
         v, f = scenes_mod.icosphere(1, 0.03, (N * H / 2,) * 3)
     else:
         v, f = _mesh(name)
-    v, f = v.astype(np.float32), f.astype(np.int32)
-    dt = np.float32(dt_scale * H / (np.sqrt(3.0) * C))
-    g = amd.PPPMSolver(N, H, dt, (0, 0, 0), 0, 0.83, C)
-    o = oracle_mod.Oracle(N, H, dt, (0, 0, 0), C, 0.83, oracle_mod.FP64)
+    v, f = (np.asarray(v, np.float64) * scale).astype(np.float32), f.astype(np.int32)
+    h = H * scale
+    dt = np.float32(dt_scale * h / (np.sqrt(3.0) * C))
+    g = amd.PPPMSolver(N, h, dt, (0, 0, 0), 0, 0.83, C)
+    o = oracle_mod.Oracle(N, h, dt, (0, 0, 0), C, 0.83, oracle_mod.FP64)
     g.set_mesh(v, f)
     o.set_mesh(v, f)
     sa, na, ra = g.get_face_weights()
