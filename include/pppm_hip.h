@@ -117,13 +117,14 @@ int pppm_run_moving(pppm_solver *s, const float *verts_series, long long vstride
  *   listen_xyz[3 (i n_listen + l) ..]; out_dev (device, steps x n_scenes x n_listen floats) gets
  *   out_dev[(k n_scenes + i) n_listen + l] = scene i's listener l after step k. use_graph != 0:
  *   32 batch steps per captured HIP graph launch. Synchronous.
- * pppm_batch_autotune: times every FDTD interior variant (0: one thread per cell; 1..4:
- *   LDS-staged 2.5D tiles of 8x64, 16x32, 4x64, 8x32 (y, z) columns) for each size class of grid
- *   edge N present in the batch (classes [0,40) [40,56) [56,72) [72,88) [88,112) [112,160)
- *   [160,...)) over `reps` repetitions, keeps the fastest per class, and (ms_out optional,
- *   7 x 5 floats) reports the milliseconds per repetition [class][variant] (untimed entries are
- *   left as they were). The FDTD launches it times do not advance t and rewrite the same values,
- *   so the scenes' state is unchanged.
+ * pppm_batch_autotune: times every FDTD interior variant (0: one thread per cell, beside the
+ *   far-field sums; 1..4: LDS-staged 2.5D tiles of 8x64, 16x32, 4x64, 8x32 (y, z) columns, in a
+ *   launch before them) for each size class of grid edge N present in the batch (classes [0,40)
+ *   [40,56) [56,72) [72,88) [88,112) [112,160) [160,...)) over `reps` repetitions of a step's FDTD
+ *   and far-field launches, keeps the fastest per class, and (ms_out optional, 7 x 5 floats)
+ *   reports the milliseconds per repetition, all scenes together [class][variant] (untimed
+ *   entries are left as they were). The launches it times do not advance t, rewrite the same
+ *   values and keep their far-field sums to themselves, so the scenes' state is unchanged.
  * pppm_batch_variants / pppm_batch_set_variants: the FDTD variant of each scene (n_scenes ints).
  * pppm_batch_set_timing / pppm_batch_get_timing: HIP-event timing of each phase of eagerly
  *   launched batch steps (a timed run does not use the graph): 0 FDTD (shell and interiors),

@@ -115,3 +115,34 @@ def test_batch_several_listeners_per_scene(amd, scenes_mod):
         g.run(torch.from_numpy(sc.neumann[:steps]).cuda(), steps, lis[i], ref)
         assert _same(out[:, i, :], ref.cpu().numpy()), (i, sc.name)
     assert np.abs(out[:, :, :2]).max() > 0
+
+
+def test_autotune_times_the_step_and_leaves_the_scenes(amd, scenes_mod):
+    """The tuner times the launches that a step makes, far-field sums beside the FDTD: on one small
+    grid a mesh of 20480 triangles takes it longer than one of 80, which the FDTD alone would not.
+    In the middle of a step (far field solved, Dirichlet update to come) it changes nothing."""
+    scs = [scenes_mod.c3_scene(24, lv, seed=3, steps=8) for lv in (1, 5)]
+    best = []
+    for sc in scs:
+        a, b = (amd.PPPMSolver(sc.res, sc.dl, sc.dt, sc.min_pos, 0, 0.83, sc.c) for _ in range(2))
+        for g in (a, b):
+            g.set_mesh(sc.verts, sc.tris)
+        for i in range(8):
+            for g in (a, b):
+                g.fdtd_step()
+                g.solve_fdtd_far()
+            if i == 5:
+                table = amd.PPPMBatch([b]).autotune(reps=20)
+                best.append(min(table[0].values()))
+            for g in (a, b):
+                g.set_neumann_condition(sc.neumann[i])
+                g.update_dirichlet()
+                g.solve_fdtd_near()
+        assert a.time_idx() == b.time_idx()
+        for rel in (0, -1):
+            assert _same(a.get_grid(rel), b.get_grid(rel))
+        for x, y in zip(a.get_history(), b.get_history()):
+            assert _same(x, y)
+        assert np.abs(a.get_grid(0)).max() > 0
+    print(f"autotune, 24^3: {1e3 * best[0]:.1f} us with 80 triangles, {1e3 * best[1]:.1f} us with 20480", flush=True)
+    assert best[1] > 1.5 * best[0]
