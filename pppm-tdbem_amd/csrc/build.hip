@@ -63,15 +63,6 @@ __global__ __launch_bounds__(B) void k_fill_int(int *__restrict__ a, long long n
         a[i] = value;
 }
 
-// copies vertex row (t - t0) of a device series into the working vertex buffer
-__global__ __launch_bounds__(B) void k_copy_verts(const float *__restrict__ series, long long stride, int t0,
-                                                  const StepState *__restrict__ st, float *__restrict__ verts, int n)
-{
-    const int i = blockIdx.x * B + threadIdx.x;
-    if (i < n)
-        verts[i] = series[(size_t)(st->t + 1 - t0) * stride + i];
-}
-
 // insertion sort of each non-empty cell's (short) list -> ascending triangle index;
 // the triangle that drew rank 0 in the fill owns the sort of its cell
 __global__ __launch_bounds__(B) void k_sort_cells(const TriGeom *__restrict__ geom, int nt,
@@ -506,12 +497,6 @@ hipError_t launch_fill_int(int *a, long long n, int value, hipStream_t s)
     if (n <= 0)
         return hipSuccess;
     k_fill_int<<<nblk(n), B, 0, s>>>(a, n, value);
-    return hipGetLastError();
-}
-hipError_t launch_copy_verts(const float *series, long long stride, int t0, const StepState *st, float *verts, int n,
-                             hipStream_t s)
-{
-    k_copy_verts<<<nblk(n), B, 0, s>>>(series, stride, t0, st, verts, n);
     return hipGetLastError();
 }
 hipError_t launch_sort_cells(const TriGeom *geom, int nt, const int *start, int *items, const int *rank,

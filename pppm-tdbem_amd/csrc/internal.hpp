@@ -145,8 +145,6 @@ struct WordRanges
     }
 };
 hipError_t launch_word_ranges(const WordRanges &r, hipStream_t s);
-hipError_t launch_copy_verts(const float *series, long long stride, int t0, const StepState *st, float *verts, int n,
-                             hipStream_t s);
 // per-tile counts of the dirty face pairs, accumulated by the face lookup for the face-pair scan
 // (layout of scan_batch_layout; zero between updates: k_tri_update clears them)
 struct TileSums

@@ -309,13 +309,12 @@ bool fork_update(const pppm_solver *s)
     return cs == hipStreamCaptureStatusNone;
 }
 
-// Geometry, binning, lists and weight caches for the vertex positions in s->verts (or, with
-// a series, row t+1-t0 of it). Asynchronous: only kernels are enqueued. The grid-cache
+// Geometry, binning, lists and weight caches for the vertex positions in s->verts, or those of
+// vsrc, which are copied there. Asynchronous: only kernels are enqueued. The grid-cache
 // recompute needs only the first scan batch (its dirty-triangle list); forked, it runs on the
 // second stream while the lists and the face cache are built, and the handle's stream waits
 // for it at the end (the step kernels read both caches).
-int enqueue_rebuild(pppm_solver *s, bool first, const float *verts_series, long long vstride, int t0,
-                    const float *vsrc = nullptr, bool use_prev = false)
+int enqueue_rebuild(pppm_solver *s, bool first, const float *vsrc, bool use_prev)
 {
     const int N = s->N, nt = s->nt;
     const int NN = N * N * N;
@@ -323,8 +322,6 @@ int enqueue_rebuild(pppm_solver *s, bool first, const float *verts_series, long 
     int *stp = s->status.p;
     int *err = stp + ST_ERR;
 
-    if (verts_series)
-        CK(launch_copy_verts(verts_series, vstride, t0, s->state.p, s->verts.p, s->nv * 3, st));
     UpdateCounters cn{s->counters.p, s->counters.p + NN, s->counters.p + 2 * NN, s->counters.p + 3 * NN, {}};
 
     // the update's three scan batches (capacity-sized, so their tile layouts are host-known);
@@ -517,7 +514,7 @@ int enqueue_attempt(pppm_solver *s, bool first, const float *vsrc, bool use_prev
         CK(launch_fill_u64(s->hkeys.p, s->hcap, ~0ull, s->stream));
         CK(launch_fill_int(s->status.p + ST_POOL, 1, 0, s->stream));
     }
-    return enqueue_rebuild(s, first, nullptr, 0, 0, vsrc, use_prev);
+    return enqueue_rebuild(s, first, vsrc, use_prev);
 }
 
 // synchronous update attempts a0..2 (used by set_mesh / update_mesh): runs the sequence, reads
@@ -898,7 +895,7 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
         return PPPM_OK;
     if (!verts_series)
         RC(ensure_ordered(s));
-    // a listener's C3 index can change with the lists: moving runs read the grid directly
+    // a listener's C3 index can change with the lists: moving runs look it up per step, not in this table
     RC(set_listeners(s, listen_xyz, n_listen));
     if (verts_series && n_listen > 0)
     {
@@ -908,31 +905,15 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
     }
     float *out = n_listen > 0 ? out_dev : nullptr;
     const int t0 = s->t_host + 1;
-    // Moving meshes take the synchronous update of pppm_update_mesh before each step (row i
-    // of the series, status read back, capacities grown when needed). The fully
-    // asynchronous update (row picked on the device, capturable in a graph) stays off until
-    // its graph replay has been verified on the device.
-    constexpr bool kAsyncMovingStep = false;
-    if (verts_series && !kAsyncMovingStep)
+    // Moving meshes take the update of pppm_update_mesh before each step (row i of the series, its
+    // status read while the step runs, capacities grown when needed): no graph
+    if (verts_series)
         use_graph = 0;
     auto one_step = [&](int i) -> int {
         const Windows win = i == 0 ? Windows::First : Windows::Next;
-        if (verts_series && !kAsyncMovingStep)
-            // the synchronous update with its status read overlapped with the step
-            return update_and_step(s, verts_series + (size_t)i * vstride, neumann_series, t0, stride, n_listen, out, win);
         if (verts_series)
-        {
-            const int sp = span_begin(s, 4);
-            RC(enqueue_rebuild(s, false, verts_series, vstride, t0));
-            span_end(s, sp);
-        }
-        if (!verts_series)
-            return enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, out, win);
-        // with moving lists the listener is read by its own launch after the near field
-        RC(enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, nullptr, win));
-        if (out)
-            CK(launch_listen_direct(scene_step(s, own_bufs(s), nullptr, t0, stride, n_listen, out), s->stream));
-        return PPPM_OK;
+            return update_and_step(s, verts_series + (size_t)i * vstride, neumann_series, t0, stride, n_listen, out, win);
+        return enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, out, win);
     };
     if (verts_series)
     {
@@ -942,7 +923,7 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
         RC(ensure_pool(s, s->pool_count + 2 * s->cap_p4));
     }
     int done = 0;
-    if (use_graph && !verts_series)
+    if (use_graph)
     {
         // a short run (a checkpoint segment) in one graph, a long one in 32-step graphs; the
         // graph is kept for later runs with the same arguments up to the per-call rows
@@ -976,7 +957,7 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
             return rc;
         }
     }
-    else if (!use_graph)
+    else
     {
         for (; done < steps; done++)
         {
@@ -986,66 +967,6 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
                 s->t_host += done;  // the steps before this one ran
                 return rc;
             }
-            if (verts_series && kAsyncMovingStep && (done % 64 == 63 || done == steps - 1))
-            {
-                RC(read_status(s));
-                RC(status_error(s));
-                if (needs_growth(s))
-                    RC(grow(s));
-            }
-        }
-    }
-    else
-    {
-        // one captured graph holds `chunk` steps; kernels read t (and the input rows) from
-        // device memory. Event timing is not captured.
-        const bool timing = s->timing;
-        s->timing = false;
-        const int chunk = std::min(steps, 32);
-        while (done < steps)
-        {
-            hipGraph_t g = nullptr;
-            hipGraphExec_t ge = nullptr;
-            CK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-            int rc = PPPM_OK;
-            for (int i = 0; i < chunk && rc == PPPM_OK; i++)
-                rc = one_step(done + i);
-            hipError_t ee = hipStreamEndCapture(s->stream, &g);
-            if (rc || ee != hipSuccess)
-            {
-                if (g)
-                    (void)hipGraphDestroy(g);
-                s->timing = timing;
-                return rc ? rc : fail(s, PPPM_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(ee));
-            }
-            CK(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
-            bool regrow = false;
-            while (done + chunk <= steps && !regrow)
-            {
-                CK(hipGraphLaunch(ge, s->stream));
-                done += chunk;
-                if (verts_series)
-                {
-                    RC(read_status(s));
-                    RC(status_error(s));
-                    regrow = needs_growth(s);
-                }
-            }
-            CK(hipStreamSynchronize(s->stream));
-            (void)hipGraphExecDestroy(ge);
-            (void)hipGraphDestroy(g);
-            if (regrow)
-                RC(grow(s));  // buffers moved: capture again
-            else
-                break;
-        }
-        for (; done < steps; done++)
-            RC(one_step(done));
-        s->timing = timing;
-        if (verts_series)
-        {
-            RC(read_status(s));
-            RC(status_error(s));
         }
     }
     s->t_host += steps;
