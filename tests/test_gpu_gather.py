@@ -45,11 +45,19 @@ def test_list_lengths_against_the_oracle(amd, oracle_mod, n, spread):
         assert np.array_equal(a.view(np.uint32), np.asarray(b).view(np.uint32).reshape(a.shape))
 
 
-@pytest.mark.parametrize("n_scenes", [1, 3, 8])
-def test_entries_per_wave_agree(amd, scenes_mod, n_scenes):
-    """Scenes of about 8000 face entries each: alone one entry per wave, together two or four."""
+def _gran(waves):
+    """Wave-map entries a wave takes in a launch of that many (gather_gran)."""
+    return 4 if waves >= 32768 else 2 if waves >= 16384 else 1
+
+
+# edge, scenes of 5120 triangles, entries per wave of the cell gathers and of the face gather (one scene
+# has 2161 cell entries and 4000 to 9000 face entries)
+@pytest.mark.parametrize("edge,n_scenes,cells,faces", [(56, 1, 1, 1), (56, 3, 1, 2), (56, 8, 2, 4), (48, 16, 4, 4)])
+def test_entries_per_wave_agree(amd, scenes_mod, edge, n_scenes, cells, faces):
+    """Scenes together, one, two or four entries a wave, against each scene alone (one entry): samples
+    inside and outside the corrected region, grids and histories."""
     import torch
-    sc = [scenes_mod.c3_scene(56, 4, seed=i, steps=6) for i in range(n_scenes)]
+    sc = [scenes_mod.c3_scene(edge, 4, seed=i, steps=6) for i in range(n_scenes)]
 
     def solvers():
         s = [amd.PPPMSolver(x.res, x.dl, x.dt, x.min_pos, 0, 0.83, x.c) for x in sc]
@@ -58,14 +66,26 @@ def test_entries_per_wave_agree(amd, scenes_mod, n_scenes):
         return s
     rng = np.random.default_rng(1)
     acc = [torch.from_numpy(rng.standard_normal((6, len(x.tris))).astype(np.float32)).cuda() for x in sc]
-    lis = [x.listener for x in sc]
     together = solvers()
-    out = torch.zeros(6, n_scenes, device="cuda")
+    lis, w3, w4 = [], [], []
+    for s in together:
+        c3 = s.get_c3()[0]
+        q = int(c3[len(c3) // 2])
+        lis.append([(q // edge ** 2, q // edge % edge, q % edge), (7 * edge // 8,) * 3])
+        assert (lis[-1][1][0] * edge + lis[-1][1][1]) * edge + lis[-1][1][2] not in c3
+        # entries by the lists' capacities: 16 face pairs a triangle, or what a first mesh grew to
+        p4, room = s.stats()["P4"], 16 * s.nt + 1024
+        w3.append(27 * s.nt // 64 + 1)
+        w4.append((room if p4 <= room else p4 * 5 // 4 + 1024) // 64 + 1)
+    assert (_gran(sum(w3)), _gran(sum(w4))) == (cells, faces), (sum(w3), sum(w4))
+    assert all((_gran(a), _gran(b)) == (1, 1) for a, b in zip(w3, w4))
+    out = torch.zeros(6, n_scenes, 2, device="cuda")
     amd.PPPMBatch(together).run(acc, 6, lis, out)
     for i, s in enumerate(solvers()):
-        one = torch.zeros(6, 1, device="cuda")
-        s.run(acc[i], 6, [lis[i]], one)
-        assert torch.equal(one[:, 0].view(torch.int32), out[:, i].contiguous().view(torch.int32))
+        one = torch.zeros(6, 2, device="cuda")
+        s.run(acc[i], 6, lis[i], one)
+        assert torch.equal(one.view(torch.int32), out[:, i].contiguous().view(torch.int32))
+        assert one[:, 0].abs().max() > 0
         assert np.array_equal(s.get_grid(0).view(np.uint32), together[i].get_grid(0).view(np.uint32))
         for a, b in zip(s.get_history(), together[i].get_history()):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
