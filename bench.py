@@ -15,6 +15,7 @@ import argparse
 import json
 import math
 import os
+import re
 import subprocess
 import sys
 import time
@@ -94,6 +95,11 @@ def host_info():
 CALIB_MIB = 256
 
 
+def is_kernel(name, kernel):
+    """Whether a dispatch's name in a profile is that of `kernel`, a template's instance or not."""
+    return re.search(rf"(?:^|\W){re.escape(kernel)}(?:<.*?>)?(?:\(|(?:\.kd)?$)", name) is not None
+
+
 def measure_traffic(kernels, workload_args):
     """HBM bytes per step of the kernels named in `kernels` (one launch each per step; their
     per-dispatch averages are added) from two rocprofv3 counter passes over a short run of
@@ -129,7 +135,7 @@ def measure_traffic(kernels, workload_args):
                                 cvals.append(v)
                                 continue
                             for k in kernels:
-                                if k + "(" in r["Kernel_Name"] or r["Kernel_Name"].endswith(k):
+                                if is_kernel(r["Kernel_Name"], k):
                                     kvals[k].append(v)
             big = max(cvals) if cvals else 0.0
             if any(not v for v in kvals.values()) or big <= 0:
