@@ -116,7 +116,8 @@ int pppm_run_moving(pppm_solver *s, const float *verts_series, long long vstride
  *   the Neumann input of step k, strides[i] >= nt_i) and n_listen listener cells (1 to 64)
  *   listen_xyz[3 (i n_listen + l) ..]; out_dev (device, steps x n_scenes x n_listen floats) gets
  *   out_dev[(k n_scenes + i) n_listen + l] = scene i's listener l after step k. use_graph != 0:
- *   32 batch steps per captured HIP graph launch. Synchronous.
+ *   runs of 64 steps or more replay a captured HIP graph of 32 batch steps (its capture would cost
+ *   shorter ones more than it saves). Synchronous.
  * pppm_batch_autotune: times every FDTD interior variant (0: one thread per cell, beside the
  *   far-field sums; 1..4: LDS-staged 2.5D tiles of 8x64, 16x32, 4x64, 8x32 (y, z) columns, in a
  *   launch before them) for each size class of grid edge N present in the batch (classes [0,40)
@@ -128,8 +129,9 @@ int pppm_run_moving(pppm_solver *s, const float *verts_series, long long vstride
  * pppm_batch_variants / pppm_batch_set_variants: the FDTD variant of each scene (n_scenes ints).
  * pppm_batch_set_timing / pppm_batch_get_timing: HIP-event timing of each phase of eagerly
  *   launched batch steps (a timed run does not use the graph): 0 FDTD (shell and interiors),
- *   1 history windows and time advance, 2 far field, 3 Dirichlet update, 4 near field;
- *   milliseconds and launch counts accumulated since the last get (which resets them). */
+ *   1 history windows and time advance, 2 far field, 3 Dirichlet update, 4 near field. A timed
+ *   step launches them one after the other, where an untimed one runs 0 beside 2 and has 1 within 3
+ *   and 4: the phases add up to more than an untimed step takes. Milliseconds and launch counts accumulated since the last get (which resets them). */
 typedef struct pppm_batch pppm_batch;
 int pppm_batch_create(pppm_batch **out, pppm_solver *const *scenes, int n_scenes);
 int pppm_batch_destroy(pppm_batch *b);
@@ -180,8 +182,8 @@ int pppm_load_state(pppm_solver *s, const void *src_dev);
  *   pppm_batch_run's output): gout_dev[(r n_scenes + i) n_listen + l] = the cotangent of scene i's
  *   listener l (cell listen_xyz[3 (i n_listen + l) ..], host, n_listen <= 64) at forward step
  *   T-steps+1+r; grad_dev[i] (device, steps x grad_strides[i] floats, grad_strides[i] >= nt_i):
- *   scene i's gradient rows as in pppm_adjoint_run. use_graph != 0: 32 reverse batch steps per
- *   captured graph launch. Synchronous. */
+ *   scene i's gradient rows as in pppm_adjoint_run. use_graph != 0: runs of 64 steps or more
+ *   replay a captured graph of 32 reverse batch steps. Synchronous. */
 int pppm_batch_adjoint_reset(pppm_batch *b, int t_last);
 int pppm_batch_adjoint_run(pppm_batch *b, const float *gout_dev, int steps, int n_listen, const int *listen_xyz,
                            float *const *grad_dev, const long long *grad_strides, int use_graph);
@@ -220,7 +222,10 @@ int pppm_stats(pppm_solver *s, long long *out8);
  * Phases: 0 FDTD, 1 far field (+ Neumann input), 2 Dirichlet update, 3 near field,
  * 4 update_mesh, and within it 5 grid-cache recompute (k_grid_weights), 6 face-cache update
  * (lookup, dirty-pair scan, integrals), 7 geometry, binning and lists. Only eagerly launched
- * work is timed (graph replays are not).
+ * work is timed (graph replays are not). A timed step launches its phases one after the other, the
+ * history windows and the time advance in between and untimed, and its update keeps to one stream;
+ * an untimed step takes three launches (FDTD beside the far field; Dirichlet update; near field with
+ * the next windows), so the phases add up to more than it takes.
  * pppm_get_timing returns accumulated milliseconds and launch counts, then resets them.
  * pppm_get_update_work: the mesh updates completed while timing was on, with the grid-cache
  * triangles and face-cache pairs they recomputed (out3 = updates, triangles, pairs), then

@@ -1,7 +1,7 @@
 // Batched scenes: many independent PPPM scenes (solver handles with their meshes set) stepped
 // together. Each kernel of the time step is one launch over every scene's blocks (a scene
-// table in device memory gives each block its scene), and a captured HIP graph replays 32
-// such batch steps per launch. The FDTD interior of each scene uses the kernel variant picked
+// table in device memory gives each block its scene); longer runs replay a captured HIP graph of 32
+// such batch steps. The FDTD interior of each scene uses the kernel variant picked
 // for its size class by the autotuner (one thread per cell, or LDS-staged 2.5D tiles); every
 // variant gives the same bits, so the batch equals the scenes' single-scene runs bit for bit.
 //
@@ -34,7 +34,7 @@ int size_class(int N)
 // FDTD interior variant per size class before any tuning (0: one thread per cell)
 constexpr int kDefaultVariant[kClasses] = {0, 0, 0, 0, 0, 0, 0};
 
-constexpr int kGraphSteps = 32;  // steps of a captured graph
+constexpr int kGraphSteps = 32;  // steps of a captured graph; runs of fewer than two are launched step by step
 
 struct Map
 {
@@ -417,8 +417,11 @@ int pppm_batch_run(pppm_batch *b, const float *const *neumann_series, const long
         BRC(enqueue_batch_windows(b));
 
     int done = 0;
-    // a graph costs its capture and instantiation on each call, with the device idle: it pays from
-    // its second replay on (64 scenes, 32 steps, this and one wait for the set-up: 14.8 -> 14.5 ms)
+    // A graph costs its capture and instantiation on each call, with the device idle, which one replay
+    // never makes good, not for the smallest batches either (one scene of 24^3, 63 steps: launched
+    // 1.06 ms, with a graph 1.44; eight of 32^3 1.26 and 1.44; reversed 2.1 and 3.0). More replays
+    // share it (eight of 32^3, 64 steps 1.24 and 1.41, 256 steps 4.24 and 4.37 ms), and spare a busy host
+    // three launches a step.
     if (use_graph && !b->timing && steps >= 2 * kGraphSteps)
     {
         const int chunk = kGraphSteps;

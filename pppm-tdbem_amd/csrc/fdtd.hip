@@ -5,15 +5,16 @@
 // laplacian (src/algorithm/fdtd.cu:7-33), ab_condition_solve / Solve4x4Linear
 // (fdtd.cu:36-137), fdtd_boundary_kernel (fdtd.cu:139-150), pml_step_kernel (fdtd.cu:162-232).
 //
-// One launch covers the whole step: the first blocks stream the interior (indices
-// 2..N-3 in every dimension, z contiguous so a wave reads 256 B rows), the remaining
-// blocks solve the 4x4 ABC system for the index-1 / N-2 shell. Interior and shell
-// write disjoint cells of level t+1; the shell also writes the ghost layer of level t,
-// which no thread of this launch reads except the writing thread itself (masked
-// terms of its own system), so the fusion is race-free. From an interior edge of 128 cells
-// (grids beyond the Infinity Cache) the interior is instead marched along x by its own
-// launch before the shell launch (k_fdtd_march). t is read from device memory (so the
-// launches can be replayed from a graph); a one-thread kernel advances it after.
+// The first blocks stream the interior (indices 2..N-3 in every dimension, z contiguous so a
+// wave reads 256 B rows), the remaining blocks solve the 4x4 ABC system for the index-1 / N-2
+// shell. Interior and shell write disjoint cells of level t+1; the shell also writes the ghost
+// layer of level t, which no thread of the launch reads except the writing thread itself (masked
+// terms of its own system), so the fusion is race-free. Without a mesh, or with phases timed, these
+// blocks are a launch (k_fdtd_abc); in a step with a mesh they run beside the far-field sums
+// (k_step_head). From an interior edge of 128 cells (kMarchMin) the interior is instead marched along
+// x by its own launch before that (k_fdtd_march). t is read from device memory, so the launches
+// can be replayed from a graph: a step in three launches hands it on (k_dirichlet, k_near),
+// otherwise a one-thread kernel advances it.
 #include "fdtd_device.hpp"
 #include "scene_device.hpp"
 
@@ -25,7 +26,11 @@ namespace pppm_amd
 namespace
 {
 
-// interior edge (N - 4) from which the interior is marched along x instead of one thread per cell
+// Interior edge (N - 4) from which the interior is marched along x instead of one thread per cell.
+// The line dates from FDTD steps of their own. The march is a launch more in a step with a mesh and
+// has few blocks in the middle of the range; a step of 80 triangles marched / per cell: 132^3 46 / 25,
+// 141^3 47 / 28, 200^3 57 / 45, 256^3 64 / 70, 324^3 223 / 149, 400^3 291 / 254 us, so a line further
+// up would serve such steps better.
 constexpr int kMarchMin = 128;
 
 // Interior of a large grid: a block owns MTY x MTZ (y, z) columns of one chunk of x planes and

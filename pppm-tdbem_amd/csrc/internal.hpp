@@ -382,14 +382,23 @@ struct SceneStep
 // scenes of a launch together). A wave spends about as long on its start (map, descriptor, first
 // indices) and on its segments' ends as on a round of 64 pairs, so where there are waves enough to
 // fill the device several times each takes up to four entries, and where there are few, one.
-// Measured per step, 1 / 2 / 4 entries: 32^3 / 1280 triangles (1.5k entries) 21 / 24 / 31 us alone;
-// 141^3 / 20480 triangles (22k face entries) 2.71 / 2.51 / 2.58 ms for 32 steps; 64 scenes (111k
-// face, 42k C3 entries) 18.2 / 16.4 / 16.0 ms for 32 steps.
+// Maps are sized by capacity (face lists a quarter above their pairs). Per step, 1 / 2 / 4 entries:
+//   both maps   32^3 / 1280 triangles (1.5k) 21 / 24 / 31 us
+//   face map    20480 triangles in one grid: 6k 81.1 / 80.7 / 84.0, 20k 59.4 / 56.7 / 56.0,
+//               27k 66.8 / 62.7 / 66.1, 61k 130.7 / 112.5 / 113.1; scenes of 5120 together:
+//               17k 54.9 / 51.7 / 50.7, 28k 82.9 / 74.2 / 74.0, 43k 136.8 / 124.1 / 123.8, 55k 175.9 /
+//               161.1 / 160.9, 131k 364.8 / 329.8 / 326.8 us
+//   cell map    scenes of 5120 triangles together: 9k 74.0 / 74.8 / 78.5, 17k 159.1 / 160.8 / 166.0,
+//               30k 238.8 / 238.4 / 242.6, 35k 267.0 / 267.0 / 268.1, 52k 391.2 / 389.9 / 388.7 us
+// The cell gathers change little either way, so the lines are those of the face gather.
 constexpr int gather_gran(long long waves) { return waves >= 4 * 8192 ? 4 : waves >= 2 * 8192 ? 2 : 1; }
 // Whether the face far field takes a launch of its own before the Dirichlet update. Formed inside
 // it, its eight dependent loads per triangle cost the gather registers and time where the device is
 // full (64 scenes: 193 -> 169 + 11 us, 80k triangles in 64^3 grids: 399 -> 347 + 8 us); where it is
-// not, a launch more costs a step of 64^3 / 5120 triangles 4 of 25 us.
+// not, a launch more costs a step of 64^3 / 5120 triangles 4 of 25 us. Around the line, inside / by
+// a launch of its own: scenes of 5120 triangles together, 17k entries 51.6 / 52.5, 28k 74.0 / 73.9, 43k
+// 127.8 / 123.8, 55k 162.1 / 160.7 us; one grid of 20480, 27k 62.9 / 61.8, 39k 78.0 / 77.6, 61k
+// 117.0 / 113.3 us.
 constexpr bool face_far_pass(long long face_waves) { return face_waves >= 4 * 8192; }
 // history windows of the gathers: wn/wd[tri*16 + k] = ring value of time t - k, the value of tap k
 // (t: the step the gathers serve, the device time index plus 1 - back when the kernel runs: back =

@@ -466,7 +466,11 @@ int pppm_modal_run(pppm_modal *m, const float *forces, int nsamples, float *accs
     k_modal_iir<<<(m->nmodes + 63) / 64, 64 * (2 + NL), 0, m->stream>>>(m->coeff, m->state, m->nmodes, f, nsamples, m->qp, ldp);
     k_modal_q<<<nblocks((long long)m->nmodes * ns_pad), MB, 0, m->stream>>>(m->qp, ldp, m->nmodes, nsamples, ns_pad,
                                                                              m->dt, m->q, m->cap_samples);
-    // 128 x 128 tiles where every CU gets two, else 128 x 64
+    // 128 x 128 tiles where every CU gets two, else 128 x 64: fewer reads of the triangles' operand
+    // against twice the blocks to spread. The whole call at 200 modes, smaller / larger tiles: 128
+    // tiles (of 128 x 128) 35.7 / 42.1 us, 320 55.7 / 62.6, 448 70.9 / 71.0, 512 75.6 / 75.1, 1024
+    // 141 / 137, 2048 265 / 260; beyond the line either can be ahead by how full the last round of
+    // blocks is (640 90 / 97, 768 106 / 106, 1280 127 / 130, 1536 200 / 208, 2560 234 / 234)
     const long long tiles = (long long)((m->nt + TT - 1) / TT) * ((nsamples + 127) / 128);
     if (tiles >= 512)
         launch_accs<2>(m->mt, m->ldm, m->nt, m->nmodes, m->q, m->cap_samples, nsamples, accs, m->stream);

@@ -560,7 +560,8 @@ __global__ __launch_bounds__(256) void k_windows(SceneStep d, int back)
 // neither waits for the other. The gather's blocks come first (they run longest). A step is this
 // launch, the Dirichlet update and the near field; with the FDTD, the time advance and the far
 // field as launches of their own and the windows rebuilt in between it was five, and each costs a
-// small scene about 5 us. One pass of 64 steps alone: 32^3 1.39 -> 1.07 ms, 64^3 1.80 -> 1.50 ms.
+// small scene about 5 us. One pass of 64 steps alone, with the same gathers in five and in three
+// launches: 32^3 1.33 -> 1.00 ms, 64^3 1.89 -> 1.56 ms.
 __global__ __launch_bounds__(TB) void k_step_head(SceneStep d, FdtdParams p, int far_blocks, int nb_inner, StatusOut f)
 {
     static_assert(TB == BLK, "gather and FDTD blocks share the launch");
