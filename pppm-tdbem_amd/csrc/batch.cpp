@@ -397,7 +397,7 @@ int pppm_batch_run(pppm_batch *b, const float *const *neumann_series, const long
         SceneStep &d = hd[i];
         d.gran3 = gather_gran(w3);
         d.gran4 = gather_gran(w4);
-        d.fused = d.win2 = b->timing ? 0 : 1;
+        d.fused = d.win2 = d.keep_far = b->timing ? 0 : 1;  // one table for all steps: every one leaves its far field
         d.ffar = b->face_far ? s->ffar.p : nullptr;
     }
     BCK(b->descs.ensure(n));

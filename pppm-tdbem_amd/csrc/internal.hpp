@@ -352,6 +352,9 @@ struct SceneStep
     // three launches (launch_step_head, launch_dirichlet, launch_near); far holds the sums the far
     // field subtracts from the pressure, which its readers subtract themselves.
     int fused;
+    // the near field of a fused step leaves the far field in far, as the phases do that may be
+    // called on their own behind it: the last step of a series
+    int keep_far;
     // the windows of step t are at (t & 1) * 16 * nt of wn / wd and the near-field launch writes
     // those of step t + 1 to the other half; 0: one set, rewritten before every step
     int win2;

@@ -646,6 +646,13 @@ enum class Windows
     Next,
     Alone,  // builds its own and leaves none (one set of windows)
 };
+// A step's place in its series. last: no step of the series follows in the same launches (a graph's last
+// step counts as one): the far field is left for the phases that may follow
+struct Place
+{
+    Windows win;
+    bool last;
+};
 
 // one update_grid_and_face on the handle's stream; neumann is device memory (row t - t0).
 // timed: phase spans when timing is on (events are created on first use, so the
@@ -653,7 +660,7 @@ enum class Windows
 // status_event != null: the FDTD launch also copies the mesh update's status block to st_h and
 // the event is recorded right behind it (the caller has checked fused_status)
 int enqueue_step(pppm_solver *s, const StepBufs &b, const float *neumann, int t0, long long stride, int n_listen,
-                 float *out, Windows win, bool timed = true, hipEvent_t status_event = nullptr)
+                 float *out, Place place, bool timed = true, hipEvent_t status_event = nullptr)
 {
     const FdtdParams fp = fdtd_params(s);
     SceneStep d = scene_step(s, b, neumann, t0, stride, n_listen, out);
@@ -672,8 +679,9 @@ int enqueue_step(pppm_solver *s, const StepBufs &b, const float *neumann, int t0
     if (!s->use_pml && !timed)
     {
         d.fused = 1;
-        d.win2 = win != Windows::Alone;
-        if (win != Windows::Next)
+        d.keep_far = place.last;
+        d.win2 = place.win != Windows::Alone;
+        if (place.win != Windows::Next)
             CK(launch_windows(d, 0, s->stream));
         CK(launch_step_head(d, fp, status, s->stream));
         if (status_event)
@@ -716,7 +724,7 @@ int check_handle(pppm_solver *s) { return s ? PPPM_OK : PPPM_ERR_ARG; }
 // neumann: device rows (row t - t0, stride; null: the ring slot is written elsewhere); out:
 // listener samples by a direct read (may be null). The caller advances t_host when it returns OK.
 int update_and_step(pppm_solver *s, const float *vsrc, const float *neumann, int t0, long long stride, int n_listen,
-                    float *out, Windows win)
+                    float *out, Place place)
 {
     auto &c = s->stc;
     if (!c.ev_status)
@@ -737,7 +745,7 @@ int update_and_step(pppm_solver *s, const float *vsrc, const float *neumann, int
         // the lists moved with this update: the near field looks the listeners' C3 indices up
         StepBufs b = own_bufs(s);
         b.lc3 = nullptr;
-        return enqueue_step(s, b, neumann, t0, stride, n_listen, out, win, true, fused_status ? c.ev_status : nullptr);
+        return enqueue_step(s, b, neumann, t0, stride, n_listen, out, place, true, fused_status ? c.ev_status : nullptr);
     };
     RC(step());
     CK(hipEventSynchronize(c.ev_status));
@@ -875,7 +883,8 @@ int enqueue_static_chunk(void *p)
     // the windows of the first step are built before the graph is launched
     const StaticChunk &c = *static_cast<const StaticChunk *>(p);
     for (int i = 0; i < c.chunk; i++)
-        RC(enqueue_step(c.s, own_bufs(c.s), c.neumann, c.t0, c.stride, c.n_listen, c.out, Windows::Next));
+        RC(enqueue_step(c.s, own_bufs(c.s), c.neumann, c.t0, c.stride, c.n_listen, c.out,
+                        {Windows::Next, i == c.chunk - 1}));
     return PPPM_OK;
 }
 
@@ -910,10 +919,11 @@ int run_impl(pppm_solver *s, const float *verts_series, long long vstride, const
     if (verts_series)
         use_graph = 0;
     auto one_step = [&](int i) -> int {
-        const Windows win = i == 0 ? Windows::First : Windows::Next;
-        if (verts_series)
-            return update_and_step(s, verts_series + (size_t)i * vstride, neumann_series, t0, stride, n_listen, out, win);
-        return enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, out, win);
+        Place place{i == 0 ? Windows::First : Windows::Next, i == steps - 1};
+        if (!verts_series)
+            return enqueue_step(s, own_bufs(s), neumann_series, t0, stride, n_listen, out, place);
+        place.last = true;  // a later update may fail
+        return update_and_step(s, verts_series + (size_t)i * vstride, neumann_series, t0, stride, n_listen, out, place);
     };
     if (verts_series)
     {
@@ -1255,7 +1265,7 @@ int pppm_step(pppm_solver *s, const float *neumann, int on_device)
         nd = s->nstage.p;
     }
     const int t_new = s->t_host + 1;
-    RC(enqueue_step(s, own_bufs(s), nd, t_new, 0, 0, nullptr, Windows::Alone));
+    RC(enqueue_step(s, own_bufs(s), nd, t_new, 0, 0, nullptr, {Windows::Alone, true}));
     s->t_host = t_new;
     return PPPM_OK;
 }
@@ -1314,7 +1324,7 @@ int pppm_run_noalloc(pppm_solver *s, const float *neumann_series, long long stri
     const int t0 = s->t_host + 1;
     float *out = n_listen > 0 ? out_dev : nullptr;
     for (int i = 0; i < steps; i++)
-        RC(enqueue_step(s, b, neumann_series, t0, stride, n_listen, out, Windows::Alone, false));
+        RC(enqueue_step(s, b, neumann_series, t0, stride, n_listen, out, {Windows::Alone, false}, false));
     s->t_host += steps;
     return PPPM_OK;
 }
@@ -1348,7 +1358,7 @@ int pppm_update_mesh_and_step(pppm_solver *s, const float *verts, const float *n
             nd = s->nstage.p;
         }
     }
-    RC(update_and_step(s, on_device ? verts : nullptr, nd, s->t_host + 1, 0, 0, nullptr, Windows::Alone));
+    RC(update_and_step(s, on_device ? verts : nullptr, nd, s->t_host + 1, 0, 0, nullptr, {Windows::Alone, true}));
     s->t_host++;
     return PPPM_OK;
 }

@@ -501,11 +501,13 @@ struct NearGather
     }
     __device__ __forceinline__ void late()
     {
-        if (d.fused && cell < nn)
-            fv = g[cell] - fv;
+        if (d.fused)
+            fv = cell < nn ? g[cell] - fv : 0.0f;
     }
     __device__ __forceinline__ void done(int s, float acc) const
     {
+        if (d.keep_far)
+            d.far[s] = fv;  // (no other wave of the launch reads it)
         const float v = (float)((double)fv + (double)acc * 0.98);
         if (cell < nn)
             g[cell] = v;

@@ -133,3 +133,54 @@ def test_step_routes_agree(amd, scenes_mod):
     for x, y in zip(a.get_history(), b.get_history()):
         assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
     assert np.array_equal(out[-1].cpu().numpy(), b.read_cells(lis))
+
+
+@pytest.mark.parametrize("route", ["step", "run", "graph", "tail", "moving", "batch", "batch_full"])
+def test_phases_behind_a_step(amd, scenes_mod, route):
+    """The far field that a step used stays for the phases called after it: another Neumann input, the
+    Dirichlet update and the near field again, against steps made of phases. tail: six steps behind two
+    graphs of 32. batch_full: scenes enough for a face far field launch of its own."""
+    import torch
+    full = route == "batch_full"
+    steps = 70 if route == "tail" else 6
+    sc = scenes_mod.c3_scene(56, 4, seed=2, steps=6) if full else scenes_mod.c1_static_sphere(steps=6)
+    rng = np.random.default_rng(5)
+    acc = rng.standard_normal((steps + 2, len(sc.tris))).astype(np.float32)
+    dev, lis = torch.from_numpy(acc).cuda(), [sc.listener]
+    out = torch.zeros(steps, 1, device="cuda")
+
+    def solver():
+        s = amd.PPPMSolver(sc.res, sc.dl, sc.dt, sc.min_pos, 0, 0.83, sc.c)
+        s.set_mesh(sc.verts, sc.tris)
+        return s
+    a, b = solver(), solver()
+    if route == "step":
+        for i in range(6):
+            b.update_grid_and_face(acc[i])
+    elif route == "moving":
+        rows = torch.from_numpy(np.repeat(sc.verts.reshape(1, -1), 6, 0).astype(np.float32)).cuda()
+        b.run_moving(rows, dev, 6, lis, out)
+    elif route == "noalloc":
+        b.run(dev, 5, lis, out, use_graph=False)
+        b.update_grid_and_face(acc[5])
+    elif route.startswith("batch"):
+        n = 8 if full else 1
+        amd.PPPMBatch([b] + [solver() for _ in range(n - 1)]).run([dev] * n, 6, lis * n,
+                                                                 torch.zeros(6, n, device="cuda"))
+    else:
+        b.run(dev, steps, lis, out, use_graph=route != "run")
+    for i in range(steps):
+        a.fdtd_step()
+        a.solve_fdtd_far()
+        a.set_neumann_condition(acc[i])
+        a.update_dirichlet()
+        a.solve_fdtd_near()
+    for i in (steps - 1, steps, steps + 1):  # the step's own input again, then others
+        for s in (a, b):
+            s.set_neumann_condition(acc[i])
+            s.update_dirichlet()
+            s.solve_fdtd_near()
+        assert np.array_equal(a.get_grid(0).view(np.uint32), b.get_grid(0).view(np.uint32)), i
+        for x, y in zip(a.get_history(), b.get_history()):
+            assert np.array_equal(x.view(np.uint32), y.view(np.uint32)), i
+    assert np.abs(a.get_grid(0)).max() > 0
