@@ -160,9 +160,6 @@ def test_phases_behind_a_step(amd, scenes_mod, route):
     elif route == "moving":
         rows = torch.from_numpy(np.repeat(sc.verts.reshape(1, -1), 6, 0).astype(np.float32)).cuda()
         b.run_moving(rows, dev, 6, lis, out)
-    elif route == "noalloc":
-        b.run(dev, 5, lis, out, use_graph=False)
-        b.update_grid_and_face(acc[5])
     elif route.startswith("batch"):
         n = 8 if full else 1
         amd.PPPMBatch([b] + [solver() for _ in range(n - 1)]).run([dev] * n, 6, lis * n,
