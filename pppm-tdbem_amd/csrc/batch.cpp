@@ -244,7 +244,9 @@ int enqueue_batch_dirichlet(pppm_batch *b)
     return PPPM_OK;
 }
 
-int enqueue_batch_step(pppm_batch *b)
+// last: of the run, or of a graph: its near field takes the second table, whose scenes keep their far
+// field
+int enqueue_batch_step(pppm_batch *b, bool last)
 {
     if (!b->timing)
     {
@@ -252,7 +254,7 @@ int enqueue_batch_step(pppm_batch *b)
         // interiors before it), the Dirichlet update, the near field with the next windows
         BRC(enqueue_batch_head(b));
         BRC(enqueue_batch_dirichlet(b));
-        BCK(launch_batch_near(b->descs.p, b->m_near.view(), b->m_win.view(), b->stream));
+        BCK(launch_batch_near(b->descs.p + (last ? b->sc.size() : 0), b->m_near.view(), b->m_win.view(), b->stream));
         return PPPM_OK;
     }
     // a span per phase: a launch each
@@ -397,11 +399,15 @@ int pppm_batch_run(pppm_batch *b, const float *const *neumann_series, const long
         SceneStep &d = hd[i];
         d.gran3 = gather_gran(w3);
         d.gran4 = gather_gran(w4);
-        d.fused = d.win2 = d.keep_far = b->timing ? 0 : 1;  // one table for all steps: every one leaves its far field
+        d.fused = d.win2 = b->timing ? 0 : 1;
         d.ffar = b->face_far ? s->ffar.p : nullptr;
     }
-    BCK(b->descs.ensure(n));
-    BCK(hipMemcpyAsync(b->descs.p, hd.data(), n * sizeof(SceneStep), hipMemcpyHostToDevice, b->stream));
+    hd.resize(2 * (size_t)n);  // the second table, for a last step's near field
+    std::copy(hd.begin(), hd.begin() + n, hd.begin() + n);
+    for (int i = n; i < 2 * n; i++)
+        hd[i].keep_far = hd[i].fused;
+    BCK(b->descs.ensure(2 * (size_t)n));
+    BCK(hipMemcpyAsync(b->descs.p, hd.data(), 2 * (size_t)n * sizeof(SceneStep), hipMemcpyHostToDevice, b->stream));
     std::vector<int> nw(n), nf(n), nff(n), nd(n), nn(n);
     for (int i = 0; i < n; i++)
     {
@@ -430,7 +436,7 @@ int pppm_batch_run(pppm_batch *b, const float *const *neumann_series, const long
         BCK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         int rc = PPPM_OK;
         for (int i = 0; i < chunk && rc == PPPM_OK; i++)
-            rc = enqueue_batch_step(b);
+            rc = enqueue_batch_step(b, i == chunk - 1);
         const hipError_t ee = hipStreamEndCapture(b->stream, &g);
         if (rc || ee != hipSuccess)
         {
@@ -453,7 +459,7 @@ int pppm_batch_run(pppm_batch *b, const float *const *neumann_series, const long
         BCK(se);
     }
     for (; done < steps; done++)
-        BRC(enqueue_batch_step(b));
+        BRC(enqueue_batch_step(b, done == steps - 1));
     BCK(hipStreamSynchronize(b->stream));
     for (pppm_solver *s : b->sc)
         s->t_host += steps;

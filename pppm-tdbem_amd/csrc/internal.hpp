@@ -353,7 +353,7 @@ struct SceneStep
     // field subtracts from the pressure, which its readers subtract themselves.
     int fused;
     // the near field of a fused step leaves the far field in far, as the phases do that may be
-    // called on their own behind it: the last step of a series
+    // called on their own behind it: the last step of a series, or of a graph
     int keep_far;
     // the windows of step t are at (t & 1) * 16 * nt of wn / wd and the near-field launch writes
     // those of step t + 1 to the other half; 0: one set, rewritten before every step

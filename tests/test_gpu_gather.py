@@ -135,14 +135,14 @@ def test_step_routes_agree(amd, scenes_mod):
     assert np.array_equal(out[-1].cpu().numpy(), b.read_cells(lis))
 
 
-@pytest.mark.parametrize("route", ["step", "run", "graph", "tail", "moving", "batch", "batch_full"])
+@pytest.mark.parametrize("route", ["step", "run", "graph", "tail", "moving", "batch", "batch_full", "batch_tail"])
 def test_phases_behind_a_step(amd, scenes_mod, route):
     """The far field that a step used stays for the phases called after it: another Neumann input, the
     Dirichlet update and the near field again, against steps made of phases. tail: six steps behind two
-    graphs of 32. batch_full: scenes enough for a face far field launch of its own."""
+    graphs of 32 (batch_tail: none). batch_full: scenes enough for a face far field launch of its own."""
     import torch
     full = route == "batch_full"
-    steps = 70 if route == "tail" else 6
+    steps = {"tail": 70, "batch_tail": 64}.get(route, 6)
     sc = scenes_mod.c3_scene(56, 4, seed=2, steps=6) if full else scenes_mod.c1_static_sphere(steps=6)
     rng = np.random.default_rng(5)
     acc = rng.standard_normal((steps + 2, len(sc.tris))).astype(np.float32)
@@ -162,8 +162,8 @@ def test_phases_behind_a_step(amd, scenes_mod, route):
         b.run_moving(rows, dev, 6, lis, out)
     elif route.startswith("batch"):
         n = 8 if full else 1
-        amd.PPPMBatch([b] + [solver() for _ in range(n - 1)]).run([dev] * n, 6, lis * n,
-                                                                 torch.zeros(6, n, device="cuda"))
+        amd.PPPMBatch([b] + [solver() for _ in range(n - 1)]).run([dev] * n, steps, lis * n,
+                                                                 torch.zeros(steps, n, device="cuda"))
     else:
         b.run(dev, steps, lis, out, use_graph=route != "run")
     for i in range(steps):
